@@ -2,15 +2,15 @@
 // evaluated on the GPU with the same IEEE operations, in the same order, per
 // output element as the reference's CPU exact path, so the two agree bit for bit.
 //
-// Mapping. The reference runs one 32-thread block per (four-row weight group,
-// lane group). Here a 64-lane wavefront runs two such blocks side by side (lanes
-// 0-31 and 32-63); within a half, lane t is the reference's thread t and owns
-// the same 64-byte weight lines (l == t mod 32), chaining fmaf over their columns
-// in ascending order. The 32 partial sums go through LDS and are added left to
-// right by one lane per output, ((P0 + P1) + P2) + ... + P31. Built with
-// -ffp-contract=off, so only the explicit fmaf calls fuse; division and square
-// root are the correctly rounded ones. Nothing here depends on the batch: a
-// block's result depends on its own weight group and lane group only.
+// Mapping. The reference runs one 32-thread block per (four-row weight group, lane
+// group): thread t owns the 64-byte weight lines l == t mod 32, chaining fmaf over
+// their columns in ascending order, and the 32 partial sums are added left to right,
+// ((P0 + P1) + P2) + ... + P31. Here one batch lane runs two such blocks side by side
+// in a 64-lane wavefront, lane t of a half being the reference's thread t; batches
+// run the chains as fp32 MFMAs (below). Built with -ffp-contract=off, so only the
+// explicit fmaf calls fuse; division and square root are the correctly rounded ones.
+// Nothing here depends on the batch: an output depends on its own weight row and
+// batch lane only.
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -30,39 +30,24 @@ __device__ __forceinline__ float lo_half(uint32_t v) { return f32_of(v << 16); }
 __device__ __forceinline__ float hi_half(uint32_t v) { return f32_of(v & 0xFFFF0000u); }
 
 // Chain t of the dot products of one four-row weight group (wg: [col][4] bf16)
-// with LG lane groups of J lanes of x (dim-major, lane j of column c at
-// x[c * stride + j], lane group i at x + 4 * xi[i]): acc[(i * 4 + r) * J + j] for
-// lane group i, row r, lane j. Lines of 8 columns: t, t + 32, ...; each line is
-// four 16-byte words, word q holding columns k + 2q (rows 0-3 in its first two
+// with one row of x: acc[r] for row r. Lines of 8 columns: t, t + 32, ...; each line
+// is four 16-byte words, word q holding columns k + 2q (rows 0-3 in its first two
 // 32-bit halves' bf16 pairs) and k + 2q + 1 (last two) (src/kernels.cu:22-94).
-// A weight line is loaded once for the LG lane groups; every output's FMAs run
-// in the same order whatever LG is.
-template <int J, int LG>
-__device__ __forceinline__ void chain(const uint16_t* wg, const float* x, int stride, int cols, int t,
-                                      const int (&xi)[LG], float (&acc)[4 * J * LG]) {
-  static_assert(J == 4 || LG == 1, "one lane: one lane group");
+__device__ __forceinline__ void chain(const uint16_t* wg, const float* x, int cols, int t, float (&acc)[4]) {
 #pragma unroll
-  for (int e = 0; e < 4 * J * LG; ++e) acc[e] = 0.0f;
-  // Line k's weights (four 16-byte words) and x columns k .. k+7 of each lane group.
+  for (int e = 0; e < 4; ++e) acc[e] = 0.0f;
+  // Line k's weights (four 16-byte words) and x columns k .. k+7.
   struct Line {
     u32x4 v[4];
-    f32x4 xc[LG][J == 1 ? 2 : 8];
+    f32x4 xc[2];
   };
   auto load = [&](int line, Line& L) {
     const int k = line * 8;
     const u32x4* wl = reinterpret_cast<const u32x4*>(wg + static_cast<int64_t>(k) * 4);
 #pragma unroll
     for (int q = 0; q < 4; ++q) L.v[q] = wl[q];
-    if constexpr (J == 1) {
-      L.xc[0][0] = *reinterpret_cast<const f32x4*>(x + k);
-      L.xc[0][1] = *reinterpret_cast<const f32x4*>(x + k + 4);
-    } else {
-#pragma unroll
-      for (int i = 0; i < LG; ++i)
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          L.xc[i][c] = *reinterpret_cast<const f32x4*>(x + static_cast<int64_t>(k + c) * stride + 4 * xi[i]);
-    }
+    L.xc[0] = *reinterpret_cast<const f32x4*>(x + k);
+    L.xc[1] = *reinterpret_cast<const f32x4*>(x + k + 4);
   };
   auto step = [&](const Line& L) {
 #pragma unroll
@@ -72,25 +57,15 @@ __device__ __forceinline__ void chain(const uint16_t* wg, const float* x, int st
         const int c = 2 * q + h;  // column k + c
         const float w[4] = {lo_half(L.v[q][2 * h]), hi_half(L.v[q][2 * h]), lo_half(L.v[q][2 * h + 1]),
                             hi_half(L.v[q][2 * h + 1])};
-        if constexpr (J == 1) {
-          const float xc = L.xc[0][c >> 2][c & 3];
+        const float xc = L.xc[c >> 2][c & 3];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(w[r], xc, acc[r]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < LG; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                acc[(i * 4 + r) * 4 + j] = __builtin_fmaf(w[r], L.xc[i][c][j], acc[(i * 4 + r) * 4 + j]);
-        }
+        for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(w[r], xc, acc[r]);
       }
     }
   };
   // Lines t, t + 32, ... in ascending order, their loads issued NB lines at a
   // time so that a lane waits one memory round trip per batch, not per line.
-  constexpr int NB = J == 1 ? 8 : (LG <= 2 ? 2 : 1);
+  constexpr int NB = 8;
   const int lines = cols / 8;
   int line = t;
   for (; line + (NB - 1) * kChains < lines; line += NB * kChains) {
@@ -108,10 +83,6 @@ __device__ __forceinline__ void chain(const uint16_t* wg, const float* x, int st
   }
 }
 
-// Columns per slice of the sliced GEMM below: 32 lines of 8, so a slice holds
-// exactly one line of each chain.
-constexpr int kSlice = 256;
-
 // ---------------------------------------------------------------------------
 // GEMM-shaped operators: Op supplies the weight group(s) of a block and the
 // epilogue on the folded sums y[m][r * J + j].
@@ -120,7 +91,6 @@ struct ResidualOp {  // src/kernels.cu:294-325
   using Params = StrideGemmResidualParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.m.groups; }
-  static bool cols_sliced(const Params& p) { return p.m.cols % kSlice == 0; }
   __device__ static const uint16_t* w(const Params& p, int, int group, int& cols) {
     cols = p.m.cols;
     return p.m.w + static_cast<int64_t>(group) * p.m.cols * 4;
@@ -138,7 +108,6 @@ struct Mlp13Op {  // src/kernels.cu:329-363
   using Params = StrideMlp13Params;
   static constexpr int kMats = 2;
   static int groups(const Params& p) { return p.w1.groups; }
-  static bool cols_sliced(const Params& p) { return p.w1.cols % kSlice == 0 && p.w3.cols == p.w1.cols; }
   __device__ static const uint16_t* w(const Params& p, int m, int group, int& cols) {
     const StrideGemmMat& mm = m == 0 ? p.w1 : p.w3;
     cols = mm.cols;
@@ -156,7 +125,6 @@ struct LmFullOp {  // src/kernels.cu:427-452
   using Params = StrideLmFullParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.m.groups; }
-  static bool cols_sliced(const Params& p) { return p.m.cols % kSlice == 0; }
   __device__ static const uint16_t* w(const Params& p, int, int group, int& cols) {
     cols = p.m.cols;
     return p.m.w + static_cast<int64_t>(group) * p.m.cols * 4;
@@ -173,7 +141,6 @@ struct LmGreedyOp {  // src/kernels.cu:383-425
   using Params = StrideLmGreedyParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.m.groups; }
-  static bool cols_sliced(const Params& p) { return p.m.cols % kSlice == 0; }
   __device__ static const uint16_t* w(const Params& p, int, int group, int& cols) {
     cols = p.m.cols;
     return p.m.w + static_cast<int64_t>(group) * p.m.cols * 4;
@@ -202,7 +169,6 @@ struct QkvOp {  // src/kernels.cu:204-284
   using Params = StrideQkvParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.q.groups + 2 * p.k.groups; }
-  static bool cols_sliced(const Params& p) { return p.q.cols % kSlice == 0; }  // k and v: the same cols
   __device__ static const uint16_t* w(const Params& p, int, int gi, int& cols) {
     const StrideGemmMat& m = gi < p.q.groups ? p.q : (gi < p.q.groups + p.k.groups ? p.k : p.v);
     const int group = gi < p.q.groups ? gi : (gi < p.q.groups + p.k.groups ? gi - p.q.groups : gi - p.q.groups - p.k.groups);
@@ -248,187 +214,272 @@ struct QkvOp {  // src/kernels.cu:204-284
   }
 };
 
-// Two blocks per 64-lane workgroup: block = 2 * (logical workgroup) + half. A
-// block is one reference block (one weight group, one lane group) for LG = 1, or
-// the reference blocks of one weight group and LG consecutive lane groups, which
-// then share each weight line load: (weight group, lane-group set) = (block /
-// sets, block % sets). The hardware hands workgroup i to XCD i % 8; logical
-// workgroups are numbered so that consecutive ones (the lane groups of one
-// weight group) share an XCD and so read that group's weights through one L2.
+// The hardware hands workgroup i to XCD i % 8; logical workgroups are numbered so
+// that consecutive ones (the lane blocks of one row block) share an XCD and so read
+// that block's weights through one L2.
 __device__ __forceinline__ int exact_wg_order(int i, int n) {
   const int full = n & ~7;
   if (i >= full) return i;
   return (i & 7) * (full >> 3) + (i >> 3);
 }
 
-template <class Op, int J, int LG>
-__global__ __launch_bounds__(64) void k_exact_gemm(typename Op::Params p, int nblocks) {
+// One batch lane (J = 1): two reference blocks (weight groups) per 64-lane workgroup,
+// group = 2 * (logical workgroup) + half. Bound by the weight stream.
+template <class Op>
+__global__ __launch_bounds__(64) void k_exact_gemm(typename Op::Params p, int ngroups) {
   constexpr int M = Op::kMats;
-  constexpr int NO = 4 * J;  // outputs per reference block
-  __shared__ float part[2][kChains][M][NO * LG];
-  __shared__ float ys[2][LG][M][16];
+  __shared__ float part[2][kChains][M][4];
+  __shared__ float ys[2][M][16];
   const int half = threadIdx.x >> 5, t = threadIdx.x & 31;
-  const int block = exact_wg_order(blockIdx.x, gridDim.x) * 2 + half;
-  const bool live = block < nblocks;
-  const int sets = (p.l.lane_groups + LG - 1) / LG;
-  const int set = live ? block % sets : 0;
-  const int group = live ? block / sets : 0;
-  const int lg0 = set * LG, nlg = min(LG, p.l.lane_groups - lg0);
+  const int group = exact_wg_order(blockIdx.x, gridDim.x) * 2 + half;
+  const bool live = group < ngroups;
   if (live) {
-    const float* x = J == 1 ? p.x : p.x + lg0 * 4;
-    int xi[LG];  // lane groups past the last live one read the last live one's x
-#pragma unroll
-    for (int i = 0; i < LG; ++i) xi[i] = min(i, nlg - 1);
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       int cols = 0;
       const uint16_t* wg = Op::w(p, m, group, cols);
-      float acc[NO * LG];
-      chain<J, LG>(wg, x, p.l.stride, cols, t, xi, acc);
+      float acc[4];
+      chain(wg, p.x, cols, t, acc);
 #pragma unroll
-      for (int e = 0; e < NO * LG; ++e) part[half][t][m][e] = acc[e];
+      for (int e = 0; e < 4; ++e) part[half][t][m][e] = acc[e];
     }
   }
   __syncthreads();
-  if (live) {
-    for (int e = t; e < NO * LG; e += kChains) {
+  if (live && t < 4) {
 #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        float y = part[half][0][m][e];
-        for (int i = 1; i < kChains; ++i) y = y + part[half][i][m][e];
-        ys[half][e / NO][m][e % NO] = y;
-      }
+    for (int m = 0; m < M; ++m) {
+      float y = part[half][0][m][t];
+      for (int i = 1; i < kChains; ++i) y = y + part[half][i][m][t];
+      ys[half][m][t] = y;
     }
   }
   __syncthreads();
-  if (live)
-    for (int i = 0; i < nlg; ++i) Op::template finish<J>(p, group, lg0 + i, t, ys[half][i]);
+  if (live) Op::template finish<1>(p, group, 0, t, ys[half]);
 }
 
-// Sliced form (four batch lanes per reference block, columns a multiple of
-// kSlice): a workgroup of NWV waves runs NB = 2 * NWV reference blocks, i.e. NB
-// consecutive weight groups with one set of LG lane groups, so the blocks share
-// x. K is taken kSlice columns at a time: slice s holds line 32 * s + t of chain
-// t, so each lane still chains its lines in ascending order and every output's
-// operations are those of chain() (and of the reference). The slice's x is
-// staged once per workgroup in LDS (double buffered, the next slice's loads in
-// flight while the current one is summed), laid out so that lane t's reads of a
-// column are consecutive 16-byte words; each lane loads its own weight line one
-// slice ahead. The matrices of a paired GEMM are swept one after the other, and
-// each one's partials are folded and finished as in k_exact_gemm.
-template <class Op, int LG, int NWV>
-__global__ __launch_bounds__(64 * NWV) void k_exact_gemm_s(typename Op::Params p, int nsets, int ngroups) {
+// Matrix form (four batch lanes per reference block). v_mfma_f32_16x16x4_f32 adds
+// its four products one after the other, k ascending, each with one rounding: the
+// same bits as four fmaf calls, denormals, signed zeros and infinities included
+// (tests/test_gpu_kat.py checks it on the device). A chain of the reference is
+// therefore a chain of MFMAs over its columns, at twice the rate of v_fma_f32
+// (155 against 78 TFLOP/s).
+//
+// A workgroup of WC waves owns NG = 4 * R weight groups (16 * R rows) and 16 * L
+// batch lanes. The 32 chains are dealt to the waves, CH neighbours at a time (two
+// neighbours read whole 128-byte lines); a wave takes its chains for all rows and
+// lanes of the tile, so a weight line and an x column are loaded once per
+// workgroup. Every CPR turns of the waves their partials meet in LDS and are added
+// left to right, ((P0 + P1) + P2) + ..., by the thread that keeps the output.
+//
+// Operands. A weight line holds 8 columns x 4 rows of a group (64 bytes): four lanes
+// load it, 16 bytes (two columns) each, one batch of four lines ahead. A batch then
+// goes through the wave's own LDS slot to reach the operand layout (lane l: row
+// l % 16, column 4s + l / 16 of step s); with R row tiles a lane reads its R rows of
+// one column as one 2R-byte word, tile r holding row r of the word. x columns are
+// loaded in operand layout directly (lane l: column 4s + l / 16, batch lanes
+// L * (l % 16) .. + L - 1 as one word, tile b holding lane b of the word).
+//
+// Bounds: few rows, the weight stream; many, the matrix pipe, which vector
+// instructions stall (an fp32 MFMA and a vector instruction share the fp32 units:
+// four v_add per four MFMAs take a bare MFMA loop from 154 to 136 TFLOP/s), so
+// larger tiles win where there are enough of them. Against fmaf chains on the vector
+// pipe, same box: N = 3072, K = 2048 at 8 / 32 / 256 rows 11.8 / 16.1 / 65 -> 7.3 /
+// 9.8 / 38 us; 2048 x 8192 34 / 40 / 162 -> 18.1 / 20.0 / 79 us (109 TFLOP/s);
+// 2 x 8192 x 2048 22.6 / 54 / 318 -> 18.1 / 27 / 177 us; 128256 x 2048 at 8 / 32 rows
+// 113 / 354 -> 108 / 184 us.
+template <int N>
+struct FloatsOf;
+template <> struct FloatsOf<1> { typedef float T; };
+template <> struct FloatsOf<2> { typedef f32x2 T; };
+template <> struct FloatsOf<4> { typedef f32x4 T; };
+
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <class Op, int R, int L, int WC, int CH, int CPR>
+__global__ __launch_bounds__(64 * WC) void k_exact_gemm_m(typename Op::Params p, int nlb, int ngroups) {
   constexpr int M = Op::kMats;
-  constexpr int NB = 2 * NWV;
-  constexpr int NO = 16;                     // outputs per reference block (4 rows x 4 lanes)
-  constexpr int XS = kSlice * LG;            // staged f32x4 per slice: one per column and lane group
-  constexpr int NT = 64 * NWV;
-  constexpr int XPER = (XS + NT - 1) / NT;   // staging loads per thread
-  __shared__ f32x4 xs[2 * XS];
-  __shared__ float part[NB][kChains][NO * LG];
-  __shared__ float ys[NB][LG][M][16];
-  const int tid = threadIdx.x, wave = tid >> 6, half = (tid >> 5) & 1, t = tid & 31;
-  const int b = wave * 2 + half;
+  constexpr int NG = 4 * R;              // weight groups per workgroup
+  constexpr int LL = 4 / R;              // lines one wave load covers (NG groups x LL lines x 4 pieces)
+  constexpr int RT = R * M;              // row tiles, over the matrices
+  constexpr int NL = 4 / CH;             // lines of each chain in a batch
+  constexpr int PC = WC * CH * CPR;      // chains folded per round
+  constexpr int NT = 64 * WC;
+  constexpr int ITEMS = RT * L * 256;    // outputs of the workgroup
+  constexpr int PER = (ITEMS + NT - 1) / NT;
+  static_assert(kChains % PC == 0, "whole rounds");
+  typedef typename FloatsOf<L>::T XV;
+  __shared__ u32x4 aw[WC][M * R * 64];
+  __shared__ float part[PC][ITEMS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w = exact_wg_order(blockIdx.x, gridDim.x);
-  const int set = w % nsets;
-  const int group = (w / nsets) * NB + b;
-  const bool live = group < ngroups;
-  const int lg0 = set * LG, nlg = min(LG, p.l.lane_groups - lg0);
+  const int g0 = (w / nlb) * NG, lg0 = (w % nlb) * 4 * L;
+  const int i = lane & 15, q = lane >> 4;
 
-  // Staging: item q of a slice is column c = q / LG, lane group q % LG (clamped
-  // to the last live one); column 8 * l + e (line l, column e of the line) sits
-  // at (e * 32 + l) * LG + i.
-  f32x4 xr[XPER];
-  auto load_x = [&](int sl) {
+  // This lane's piece of a wave load: group pg, line slot pl, piece kp of the line.
+  const int pg = lane / (4 * LL), pl = (lane >> 2) % LL, kp = lane & 3;
+  const uint16_t* wp[M];
+  int cols = 0;
 #pragma unroll
-    for (int r = 0; r < XPER; ++r) {
-      const int q = tid + r * NT;
-      if (q < XS) {
-        const int c = q / LG, i = min(q % LG, nlg - 1);
-        xr[r] = *reinterpret_cast<const f32x4*>(p.x + static_cast<int64_t>(sl * kSlice + c) * p.l.stride + 4 * (lg0 + i));
-      }
-    }
-  };
-  auto store_x = [&](int buf) {
+  for (int m = 0; m < M; ++m) wp[m] = Op::w(p, m, min(g0 + pg, ngroups - 1), cols) + kp * 8;
+  const int lines = cols / 8;
+  const int stride = p.l.stride;
+  uint32_t xo[2];  // this lane's byte offset from column 0 of a line: columns q and 4 + q
 #pragma unroll
-    for (int r = 0; r < XPER; ++r) {
-      const int q = tid + r * NT;
-      if (q < XS) {
-        const int c = q / LG, i = q % LG, l = c >> 3, e = c & 7;
-        xs[buf * XS + (e * 32 + l) * LG + i] = xr[r];
-      }
-    }
-  };
+  for (int s = 0; s < 2; ++s) xo[s] = 4u * (static_cast<uint32_t>(4 * s + q) * stride + min(lg0 * 4 + L * i, stride - L));
+  const int per_chain = (lines + kChains - 1) / kChains;  // lines of chain 0, the longest
+  const int nb = (per_chain + NL - 1) / NL;               // batches
 
-  unroll<M>([&](auto mm) {
-    constexpr int m = decltype(mm)::value;
-    int cols = 0;
-    const uint16_t* wg = Op::w(p, m, min(group, ngroups - 1), cols);
-    const int nsl = cols / kSlice;
-    u32x4 wl[2][4];  // this lane's weight line of the current and the next slice
-    auto load_w = [&](int sl, auto buf) {
-      const u32x4* src = reinterpret_cast<const u32x4*>(wg + static_cast<int64_t>(sl * kChains + t) * 32);
+  // Slot n of a batch: line n / CH of the batch in chain t + n % CH. Slots past a
+  // chain's last line are loaded from the matrix's last line and not summed.
+  struct Batch {
+    u32x4 a[M][R];
+    XV x[4][2];
+  };
+  auto line_of = [&](int t, int b, int n) { return t + n % CH + kChains * (b * NL + n / CH); };
+  auto load = [&](int t, int b, Batch& B) __attribute__((always_inline)) {
+    unroll<R>([&](auto rr) {
+      constexpr int r = decltype(rr)::value;
+      const int64_t line = min(line_of(t, b, r * LL + pl), lines - 1);
+      unroll<M>([&](auto mm) {
+        constexpr int m = decltype(mm)::value;
+        B.a[m][r] = load16(wp[m] + line * 32);
+      });
+    });
+    unroll<4>([&](auto nn) {
+      constexpr int n = decltype(nn)::value;
+      const int64_t line = min(line_of(t, b, n), lines - 1);
+      const char* base = reinterpret_cast<const char*>(p.x + line * 8 * stride);
+      B.x[n][0] = *reinterpret_cast<const XV*>(base + xo[0]);
+      B.x[n][1] = *reinterpret_cast<const XV*>(base + xo[1]);
+    });
+  };
+  f32x4 acc[CH][RT][L];
+  auto slot_step = [&](const Batch& B, auto nn) __attribute__((always_inline)) {
+    constexpr int n = decltype(nn)::value;
+    unroll<2>([&](auto ss) {
+      constexpr int s = decltype(ss)::value;
+      float av[RT];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) wl[decltype(buf)::value][q] = src[q];
-    };
-    float acc[NO * LG];
-#pragma unroll
-    for (int e = 0; e < NO * LG; ++e) acc[e] = 0.0f;
-    auto step = [&](auto buf) {
-      constexpr int c2 = decltype(buf)::value;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int c = 2 * q + h;  // column c of the line
-          const float wv[4] = {lo_half(wl[c2][q][2 * h]), hi_half(wl[c2][q][2 * h]), lo_half(wl[c2][q][2 * h + 1]),
-                               hi_half(wl[c2][q][2 * h + 1])};
-#pragma unroll
-          for (int i = 0; i < LG; ++i) {
-            const f32x4 xc = xs[c2 * XS + (c * 32 + t) * LG + i];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-              for (int j = 0; j < 4; ++j) acc[(i * 4 + r) * 4 + j] = __builtin_fmaf(wv[r], xc[j], acc[(i * 4 + r) * 4 + j]);
-          }
+      for (int m = 0; m < M; ++m) {
+        const char* src = reinterpret_cast<const char*>(&aw[wave][m * R * 64 + (n * 4 + 2 * s + (q >> 1)) * NG]) + (q & 1) * 8;
+        if constexpr (R == 1) {
+          av[m] = lo_half(*reinterpret_cast<const uint16_t*>(src + (i >> 2) * 16 + (i & 3) * 2));
+        } else if constexpr (R == 2) {
+          const uint32_t v = *reinterpret_cast<const uint32_t*>(src + (i >> 1) * 16 + (i & 1) * 4);
+          av[m * R] = lo_half(v);
+          av[m * R + 1] = hi_half(v);
+        } else {
+          const u32x2 v = *reinterpret_cast<const u32x2*>(src + i * 16);
+          av[m * R] = lo_half(v[0]);
+          av[m * R + 1] = hi_half(v[0]);
+          av[m * R + 2] = lo_half(v[1]);
+          av[m * R + 3] = hi_half(v[1]);
         }
       }
-    };
-    load_x(0);
-    load_w(0, std::integral_constant<int, 0>{});
-    store_x(0);
-    __syncthreads();
-    // Slices in pairs so that the register and LDS buffers are compile-time.
-    // The next slice's loads are issued unconditionally (the last slice's again
-    // after it, into buffers nobody reads), so every pass waits on the same loads.
-    int sl = 0;
-    auto one = [&](auto cur) {
-      constexpr int c = decltype(cur)::value;
-      const int nx = min(sl + 1, nsl - 1);
-      load_x(nx);
-      load_w(nx, std::integral_constant<int, c ^ 1>{});
-      step(cur);
-      store_x(c ^ 1);
-      __syncthreads();
-      ++sl;
-    };
-    while (sl < nsl) {
-      one(std::integral_constant<int, 0>{});
-      if (sl < nsl) one(std::integral_constant<int, 1>{});
+      unroll<L>([&](auto bb) {
+        constexpr int b = decltype(bb)::value;
+        float xv;
+        if constexpr (L == 1) xv = B.x[n][s];
+        else xv = B.x[n][s][b];
+        unroll<RT>([&](auto rr) {
+          constexpr int r = decltype(rr)::value;
+          acc[n % CH][r][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[r], xv, acc[n % CH][r][b], 0, 0, 0);
+        });
+      });
+    });
+  };
+  // One batch: through the LDS slot (pieces at (line slot, piece, group), so that an
+  // operand read touches consecutive words), then eight steps.
+  auto sum = [&](const Batch& B, int t, int b) __attribute__((always_inline)) {
+    unroll<M * R>([&](auto ee) {
+      constexpr int m = decltype(ee)::value / R, r = decltype(ee)::value % R;
+      aw[wave][m * R * 64 + ((r * LL + pl) * 4 + kp) * NG + pg] = B.a[m][r];
+    });
+    if (line_of(t, b, 3) < lines) {
+      unroll<4>([&](auto n) { slot_step(B, n); });
+    } else {
+      if (line_of(t, b, 0) < lines) slot_step(B, std::integral_constant<int, 0>{});
+      if (line_of(t, b, 1) < lines) slot_step(B, std::integral_constant<int, 1>{});
+      if (line_of(t, b, 2) < lines) slot_step(B, std::integral_constant<int, 2>{});
     }
-    // Partials of this matrix, folded left to right per output.
-#pragma unroll
-    for (int e = 0; e < NO * LG; ++e) part[b][t][e] = acc[e];
-    __syncthreads();
-    for (int e = t; e < NO * LG; e += kChains) {
-      float y = part[b][0][e];
-      for (int i = 1; i < kChains; ++i) y = y + part[b][i][e];
-      ys[b][e / NO][m][e % NO] = y;
-    }
-    __syncthreads();
+  };
+  unroll<CH * RT * L>([&](auto ee) {
+    constexpr int e = decltype(ee)::value;
+    acc[e / (RT * L)][e / L % RT][e % L] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   });
-  if (live)
-    for (int i = 0; i < nlg; ++i) Op::template finish<4>(p, group, lg0 + i, t, ys[b][i]);
+
+  // Turn n of a wave: chains (n * WC + wave) * CH ..; a round is CPR turns of every
+  // wave, whose partials are then added to the outputs, chains ascending.
+  float y[PER];
+  constexpr int kTurns = kChains / (WC * CH);
+  auto first_chain = [&](int turn) { return (turn * WC + wave) * CH; };
+  auto end_turn = [&](int turn) __attribute__((always_inline)) {
+    const int in_round = turn % CPR;
+    if (turn > 0 && in_round == 0) lds_barrier();  // the last round's partials have been read
+    unroll<CH * RT * L>([&](auto ee) {
+      constexpr int e = decltype(ee)::value, c = e / (RT * L);
+      f32x4& a = acc[c][e / L % RT][e % L];
+      reinterpret_cast<f32x4*>(part[(in_round * WC + wave) * CH + c])[e % (RT * L) * 64 + lane] = a;
+      a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    });
+    if (in_round != CPR - 1) return;
+    lds_barrier();
+    unroll<PER>([&](auto uu) {
+      constexpr int u = decltype(uu)::value;
+      const int e = tid + NT * u;
+      if (ITEMS % NT == 0 || e < ITEMS) {
+        float v = turn < CPR ? part[0][e] : y[u] + part[0][e];
+#pragma unroll
+        for (int k = 1; k < PC; ++k) v = v + part[k][e];
+        y[u] = v;
+      }
+    });
+  };
+  // The next batch's loads are in flight while one is summed.
+  Batch B[2];
+  load(first_chain(0), 0, B[0]);
+  int turn = 0, b = 0;
+  auto pass = [&](auto buf) __attribute__((always_inline)) {
+    constexpr int k = decltype(buf)::value;
+    const bool last = b == nb - 1;
+    load(first_chain(min(turn + (last ? 1 : 0), kTurns - 1)), last ? 0 : b + 1, B[k ^ 1]);
+    sum(B[k], first_chain(turn), b);
+    ++b;
+    if (last) {
+      end_turn(turn);
+      ++turn;
+      b = 0;
+    }
+  };
+  while (turn < kTurns) {
+    pass(std::integral_constant<int, 0>{});
+    if (turn < kTurns) pass(std::integral_constant<int, 1>{});
+  }
+
+  // Outputs back to (group, lane group) blocks of sixteen, then the operator's finish.
+  lds_barrier();
+  float* ys = &part[0][0];  // [NG * 4 * L][M][16]
+  unroll<PER>([&](auto uu) {
+    constexpr int u = decltype(uu)::value;
+    const int e = tid + NT * u;
+    if (ITEMS % NT == 0 || e < ITEMS) {
+      const int tile = e >> 8, b_ = tile % L, rt = tile / L, m = rt / R, r = rt % R;
+      const int ln = (e & 255) >> 2, row = 4 * (ln >> 4) + (e & 3), bl = L * (ln & 15) + b_;
+      const int g = row * R / 4, rr = (row * R) % 4 + r;
+      ys[((g * 4 * L + (bl >> 2)) * M + m) * 16 + rr * 4 + (bl & 3)] = y[u];
+    }
+  });
+  lds_barrier();
+  for (int k = tid >> 4; k < NG * 4 * L; k += NT / 16) {
+    const int group = g0 + k / (4 * L), lg = lg0 + k % (4 * L);
+    if (group < ngroups && lg < p.l.lane_groups)
+      Op::template finish<4>(p, group, lg, tid & 15, reinterpret_cast<const float(*)[16]>(ys + k * M * 16));
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -676,30 +727,54 @@ int launched(const char* what) {
   return 0;
 }
 
-#ifndef STRIDE_EXACT_LG
-#define STRIDE_EXACT_LG 2
-#endif
+template <class Op, int R, int L, int WC, int CH, int CPR>
+int run_matrix(const typename Op::Params& p, hipStream_t st, const char* what) {
+  const int nlb = (p.l.lane_groups + 4 * L - 1) / (4 * L);
+  const int nrb = (Op::groups(p) + 4 * R - 1) / (4 * R);
+  hipLaunchKernelGGL((k_exact_gemm_m<Op, R, L, WC, CH, CPR>), dim3(nrb * nlb), dim3(64 * WC), 0, st, p, nlb, Op::groups(p));
+  return launched(what);
+}
+
 template <class Op>
 int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what) {
-  constexpr int LG = STRIDE_EXACT_LG;  // lane groups sharing a weight line load
-  const int lg = J == 1 ? 1 : LG;
-  const int nblocks = Op::groups(p) * ((p.l.lane_groups + lg - 1) / lg);
-  if (p.l.rows == 0 || nblocks == 0) return 0;
+  const int groups = Op::groups(p);
+  if (p.l.rows == 0 || groups == 0) return 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // Four batch lanes per reference block: the sliced form shares x over eight
-  // weight groups. (One lane: the loads are weight-bound, and the streaming
-  // form keeps more of them in flight.)
-  if (J == 4 && Op::cols_sliced(p)) {
-    constexpr int NWV = 4;
-    const int sets = (p.l.lane_groups + lg - 1) / lg;
-    const dim3 sgrid(((Op::groups(p) + 2 * NWV - 1) / (2 * NWV)) * sets);
-    hipLaunchKernelGGL((k_exact_gemm_s<Op, LG, NWV>), sgrid, dim3(64 * NWV), 0, st, p, sets, Op::groups(p));
+  // One lane: the loads are weight-bound, and the streaming form keeps more of them
+  // in flight than a matrix tile with one live lane in sixteen would.
+  if (J == 1) {
+    hipLaunchKernelGGL((k_exact_gemm<Op>), dim3((groups + 1) / 2), dim3(64), 0, st, p, groups);
     return launched(what);
   }
-  const dim3 grid((nblocks + 1) / 2);
-  if (J == 1) hipLaunchKernelGGL((k_exact_gemm<Op, 1, 1>), grid, dim3(64), 0, st, p, nblocks);
-  else hipLaunchKernelGGL((k_exact_gemm<Op, 4, LG>), grid, dim3(64), 0, st, p, nblocks);
-  return launched(what);
+  // Tile and waves by the number of 16 x 16 output tiles, from a sweep of 18 tile and
+  // wave shapes at 2-256 rows, N = 2048, 3072, 2 x 8192 and 128256, K = 2048 and 8192:
+  // the workgroups have to fill the 256 CUs, so few tiles get a workgroup of 16 waves
+  // each, many get larger tiles (fewer operand loads and vector instructions per MFMA)
+  // and smaller workgroups (more of them resident, so that one folds while another
+  // multiplies). The other side of each line, measured: 256 tiles 7.2 us at 16 waves
+  // per tile against 9.3 at two tiles per workgroup (N = K = 2048, 32 rows); 384 tiles
+  // 13.4 against 9.8 (N = 3072, 32 rows); 768 tiles 18.3 at 1 x 2 against 15.5 at 2 x 2;
+  // 1536 tiles 28.7 at 2 x 2 x 16 waves against 21.3 (128 rows); 2048 tiles 27.2 at
+  // 1 x 2 against 25.1 at 2 x 4, whose four lane tiles have to be live (K = 8192: 91
+  // against 79); 3072 tiles 48 at 2 x 4 against 38 (256 rows).
+  const int rt = (groups + 3) / 4, lt = (p.l.lane_groups + 3) / 4;
+  const int64_t tiles = static_cast<int64_t>(rt) * lt;
+  if (tiles <= 256) return run_matrix<Op, 1, 1, 16, 2, 1>(p, st, what);
+  if constexpr (Op::kMats == 2) {
+    if (lt == 1) return run_matrix<Op, 1, 1, 8, 2, 1>(p, st, what);
+    if (tiles <= 512) return run_matrix<Op, 1, 2, 16, 1, 1>(p, st, what);
+    return run_matrix<Op, 1, 2, 8, 1, 2>(p, st, what);
+  } else {
+    // One lane tile over many rows (the vocabulary): the weight stream; 4 x 1 tiles read
+    // it fastest (128256 x 2048, 8 rows: 105-108 us, 5.0 TB/s, against 118 at 2 x 1).
+    if (lt == 1)
+      return tiles >= 2048 ? run_matrix<Op, 4, 1, 4, 2, 1>(p, st, what) : run_matrix<Op, 1, 1, 8, 2, 1>(p, st, what);
+    if (tiles <= 512) return run_matrix<Op, 1, 2, 16, 2, 1>(p, st, what);
+    if (tiles <= 1024) return run_matrix<Op, 2, 2, 16, 1, 1>(p, st, what);
+    if (tiles <= 1536 || (tiles <= 2048 && lt % 4 != 0)) return run_matrix<Op, 1, 2, 8, 1, 2>(p, st, what);
+    if (tiles <= 2048) return run_matrix<Op, 2, 4, 8, 1, 1>(p, st, what);
+    return run_matrix<Op, 2, 2, 4, 2, 1>(p, st, what);
+  }
 }
 
 }  // namespace

@@ -20,6 +20,8 @@ def load():
         lib.mfma_kat_tiles.restype = C.c_int
         lib.mfma_kat_equiv.argtypes = [vp, vp, vp, vp, vp, C.c_int32, C.c_int32, vp]
         lib.mfma_kat_equiv.restype = C.c_int
+        lib.mfma_kat_f32.argtypes = [vp, vp, vp, vp, vp, C.c_int32, C.c_int32, vp]
+        lib.mfma_kat_f32.restype = C.c_int
         _lib = lib
     return _lib
 
@@ -35,3 +37,10 @@ def mfma_equiv(a, b, c0, o16, o32, chunks: int, stream: int) -> None:
                                c0.shape[0], chunks, stream)
     if rc:
         raise RuntimeError(f"mfma_kat_equiv failed ({rc})")
+
+
+def mfma_f32(a, b, c, out, want, steps: int, stream: int) -> None:
+    rc = load().mfma_kat_f32(a.data_ptr(), b.data_ptr(), c.data_ptr(), out.data_ptr(), want.data_ptr(), c.shape[0],
+                             steps, stream)
+    if rc:
+        raise RuntimeError(f"mfma_kat_f32 failed ({rc})")

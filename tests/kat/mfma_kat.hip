@@ -3,7 +3,7 @@
 // product): one v_mfma_f32_16x16x32_bf16 per tile on the packed tile layout (the
 // position-invariance test permutes rows and lanes inside a tile), and the
 // equivalence of one 16x16x32 MFMA per 32-column chunk with two chained
-// 32x32x16 MFMAs. The gfx950 counterpart of the reference's tc_probe Q1
+// 32x32x16 MFMAs; and v_mfma_f32_16x16x4_f32 as a chain of fmaf. The gfx950 counterpart of the reference's tc_probe Q1
 // (tools/tc_probe.cu:25-35, 106-139).
 #include <hip/hip_runtime.h>
 
@@ -71,7 +71,40 @@ __global__ __launch_bounds__(64) void k_mfma_equiv(const uint16_t* a, const uint
   for (int i = 0; i < 16; ++i) o32[(8 * (i / 4) + 4 * (lane / 32) + i % 4) * 32 + lane % 32] = acc[i];
 }
 
+// out = the accumulator after `steps` v_mfma_f32_16x16x4_f32 from c: one 16x16 tile
+// per workgroup, a [t][16 rows][4 * steps], b [t][4 * steps][16 lanes], c and out
+// [t][16][16], all fp32. A lane l: row l%16, k = l/16; B lane l: lane l%16, k = l/16.
+__global__ __launch_bounds__(64) void k_mfma_f32(const float* a, const float* b, const float* c, float* out, int steps) {
+  const int lane = threadIdx.x, i = lane & 15, q = lane >> 4;
+  const int64_t t = blockIdx.x;
+  a += t * 64 * steps;
+  b += t * 64 * steps;
+  f32x4 acc;
+  for (int v = 0; v < 4; ++v) acc[v] = c[t * 256 + (4 * q + v) * 16 + i];
+  for (int s = 0; s < steps; ++s)
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i * 4 * steps + 4 * s + q], b[(4 * s + q) * 16 + i], acc, 0, 0, 0);
+  for (int v = 0; v < 4; ++v) out[t * 256 + (4 * q + v) * 16 + i] = acc[v];
+}
+
+// The same products as fmaf calls, k ascending.
+__global__ __launch_bounds__(256) void k_fma_f32(const float* a, const float* b, const float* c, float* out, int steps) {
+  const int i = threadIdx.x >> 4, j = threadIdx.x & 15;
+  const int64_t t = blockIdx.x;
+  float acc = c[t * 256 + threadIdx.x];
+  for (int k = 0; k < 4 * steps; ++k)
+    acc = __builtin_fmaf(a[t * 64 * steps + i * 4 * steps + k], b[t * 64 * steps + k * 16 + j], acc);
+  out[t * 256 + threadIdx.x] = acc;
+}
+
 }  // namespace
+
+extern "C" int mfma_kat_f32(const float* a, const float* b, const float* c, float* out, float* want, int32_t tiles,
+                            int32_t steps, void* stream) {
+  if (!a || !b || !c || !out || !want || tiles <= 0 || steps <= 0) return 1;
+  hipLaunchKernelGGL(k_mfma_f32, dim3(tiles), dim3(64), 0, static_cast<hipStream_t>(stream), a, b, c, out, steps);
+  hipLaunchKernelGGL(k_fma_f32, dim3(tiles), dim3(256), 0, static_cast<hipStream_t>(stream), a, b, c, want, steps);
+  return static_cast<int>(hipGetLastError());
+}
 
 extern "C" int mfma_kat_tiles(const uint16_t* a, const uint16_t* b, const float* c, float* out, int32_t tiles,
                               void* stream) {

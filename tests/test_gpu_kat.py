@@ -74,3 +74,32 @@ def test_mfma_shapes_equivalent():
         ref = c0.double() + torch.einsum("tmk,tnk->tmn", a.double(), b.double())
         assert torch.allclose(o16.double(), ref, rtol=1e-3, atol=1e-3 * ref.abs().max().item())
         assert torch.equal(o16.view(torch.int32), o32.view(torch.int32)), f"shapes differ at chunks={chunks}"
+
+
+@pytest.mark.parametrize("lo,hi", [(0, 1), (-30, 30), (-150, -110)])
+def test_f32_mfma_is_a_chain_of_fmaf(lo, hi):
+    """v_mfma_f32_16x16x4_f32 equals four fmaf calls, k ascending, bit for bit, for
+    operands of ordinary size, over 60 binary orders of magnitude, and with
+    subnormal products; zeros of both signs and infinities are among them. The
+    exact path's batched GEMMs and the attention tiles rest on this."""
+    g = torch.Generator(device=DEV).manual_seed(7)
+    tiles, steps = 2048, 5
+
+    def draw(*shape, scaled=True):
+        t = torch.randn(*shape, generator=g, device=DEV)
+        if scaled:
+            t = torch.ldexp(t, torch.randint(lo, hi, t.shape, generator=g, device=DEV))
+        u = torch.rand(t.shape, generator=g, device=DEV)
+        t[u < 0.02] = 0.0
+        t[u > 0.98] = -0.0
+        if lo == -30:
+            t[(u > 0.5) & (u < 0.502)] = float("inf")
+        return t
+
+    a, b, c = draw(tiles, 16, 4 * steps), draw(tiles, 4 * steps, 16, scaled=lo >= -30), draw(tiles, 16, 16)
+    out, want = torch.empty_like(c), torch.empty_like(c)
+    kat.mfma_f32(a, b, c, out, want, steps, stream())
+    torch.cuda.synchronize()
+    nan = torch.isnan(want)
+    assert torch.equal(nan, torch.isnan(out))
+    assert torch.equal(out.view(torch.int32)[~nan], want.view(torch.int32)[~nan])
