@@ -293,12 +293,6 @@ template <> struct FloatsOf<1> { typedef float T; };
 template <> struct FloatsOf<2> { typedef f32x2 T; };
 template <> struct FloatsOf<4> { typedef f32x4 T; };
 
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 template <class Op, int R, int L, int WC, int CH, int CPR>
 __global__ __launch_bounds__(64 * WC) void k_exact_gemm_m(typename Op::Params p, int nlb, int ngroups) {
   constexpr int M = Op::kMats;

@@ -11,6 +11,8 @@
 // (independent positions, dimensions and lanes); sequential sums stay sequential.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <climits>
 #include <cstddef>
 #include <string>
 
@@ -204,38 +206,114 @@ __device__ __forceinline__ const KvT* kv_row(const StrideKvRef& kv, int page_shi
          which * kv.which_elems + group * kv.group_elems + static_cast<int64_t>(token) * kv.head_dim;
 }
 
+// One row's sums over a page, by one wave. Scores: lane i holds position i, and an
+// fmaf chain over the dims in order is a chain of v_mfma_f32_4x4x1_16b_f32, one per dim
+// (one fmaf per output; the query column of four heads is block `dim % 16` of the left
+// operand, given to all sixteen blocks, which hold four positions each). Mix: lane d
+// holds dim d, one MFMA per position with the four heads' weights as the column. The
+// four heads cost 8 cycles of the fp32 units a dim or position, against 16 as v_fma_f32.
+// Where the KV loads bound the kernel that shows little (bf16, 128 rows of 4-8 pages 30.1
+// -> 29.4 us), more where they do not (fp32 KV, 32 rows 16.1 -> 13.2 us; bf16, 530 rows of
+// 9 pages, each row's read again from L2, 91 -> 69 us).
+//
+// qa: lane h + 4b holds q[h][16e + b] in qa[e].
+template <int D>
+__device__ __forceinline__ void load_query(const float* qrow, int lane, float (&qa)[D / 16]) {
+#pragma unroll
+  for (int e = 0; e < D / 16; ++e) qa[e] = qrow[(lane & 3) * D + 16 * e + (lane >> 2)];
+}
+template <int D, class KvT>
+__device__ __forceinline__ f32x4 page_scores(const u32x4 (&kr)[D * sizeof(KvT) / 16], const float (&qa)[D / 16]) {
+  f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+  // Eight dims widened ahead of their MFMAs: one that reads a register written just
+  // before it waits.
+  unroll<D / 8>([&](auto cc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value;
+    float k[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (sizeof(KvT) == 2) k[e] = f32_of(e & 1 ? kr[c][e / 2] & 0xFFFF0000u : kr[c][e / 2] << 16);
+      else k[e] = f32_of(kr[2 * c + e / 4][e % 4]);
+    }
+    if constexpr (sizeof(KvT) == 2)
+      asm("" : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3]), "+v"(k[4]), "+v"(k[5]), "+v"(k[6]), "+v"(k[7]));
+    unroll<8>([&](auto ee) __attribute__((always_inline)) {
+      constexpr int e = decltype(ee)::value, d = 8 * c + e;
+      a = __builtin_amdgcn_mfma_f32_4x4x1f32(qa[d / 16], k[e], a, 4, d % 16, 0);
+    });
+  });
+  return a;
+}
+// wt: [head][position] weights; vs: the page's V rows. acc[t][h]: dim lane + 64t of head
+// h; den: head lane & 3, its weights added left to right.
+template <int D, class KvT>
+__device__ __forceinline__ void page_mix(const float* wt, const KvT (*vs)[D], int n, int lane, f32x4 (&acc)[(D + 63) / 64],
+                                         float& den) {
+  constexpr int T = (D + 63) / 64;
+#pragma unroll
+  for (int t = 0; t < T; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  den = 0.0f;
+  const float* wh = wt + (lane & 3) * kAttnPage;
+  const int d0 = min(lane, D - 1);
+  for (int i0 = 0; i0 < n; i0 += 16) {
+    const float wa = wh[i0 + (lane >> 2)];  // lane h + 4b: head h, position i0 + b
+    f32x4 wd[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wd[e] = *reinterpret_cast<const f32x4*>(wh + i0 + 4 * e);
+    float v[16][T];
+#pragma unroll
+    for (int b = 0; b < 16; ++b)
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        if constexpr (sizeof(KvT) == 2) v[b][t] = f32_of(static_cast<uint32_t>(vs[i0 + b][d0 + 64 * t]) << 16);
+        else v[b][t] = vs[i0 + b][d0 + 64 * t];
+      }
+    auto one = [&](auto bb) __attribute__((always_inline)) {
+      constexpr int b = decltype(bb)::value;
+      unroll<T>([&](auto tt) {
+        constexpr int t = decltype(tt)::value;
+        acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(wa, v[b][t], acc[t], 4, b, 0);
+      });
+      den = den + wd[b / 4][b % 4];
+    };
+    if (i0 + 16 <= n) {
+      unroll<16>(one);
+    } else {
+      unroll<16>([&](auto bb) __attribute__((always_inline)) {
+        if (i0 + decltype(bb)::value < n) one(bb);  // n is the same for every lane
+      });
+    }
+  }
+}
+
 // One (row, page) item for one KV group (src/kernel_common.h:84-250). The page's
 // V rows are fetched with 16-byte loads and parked in LDS, and each lane's K row
 // is fetched whole, so both latencies overlap. Lane i scores position p0 + i for
-// the four query heads (an fmaf chain over the head dims in order, then times
-// scale); the page maximum is order-free; the exponentials follow. Each lane
-// then mixes the values of its dims over the positions in order; in the same
-// pass lane h < 4 adds head h's weights left to right (one LDS word per
-// position), which yields the denominators without a serial phase and without
-// every lane repeating the four adds.
+// the four query heads; the page maximum is order-free; the exponentials follow, and
+// each lane then mixes the values of its dims over the positions in order.
 // KvT is uint16_t (bf16 KV, the tensor-core path) or float (the exact path);
-// the arithmetic is the same, on the widened values.
+// the arithmetic is the same, on the widened values. Taken by one wave, with LDS of its
+// own; LDS accesses of a wave are performed in order, so its phases need no waits.
 template <int D, class KvT>
-__global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int page_shift) {
+struct PageLds {
+  float wt[kHeadsPerGroup * kAttnPage];  // weights [head][position]
+  KvT vs[kAttnPage][D];
+};
+__device__ __forceinline__ void wave_phase() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+template <int D, class KvT>
+__device__ __forceinline__ void page_item(const StrideAttentionParams& p, int page_shift, int j, int page, int g, int lane,
+                                          PageLds<D, KvT>& lds) {
   constexpr int kEl = 16 / static_cast<int>(sizeof(KvT));  // elements per 16-byte piece
-  constexpr int kPieces = kAttnPage * D / kEl;  // 16-byte pieces of one page of V
-  constexpr int kPer = kPieces / 64;            // per lane
-  constexpr int kKey = D / kEl;                 // 16-byte pieces of one K row
-  const int item = blockIdx.x / p.n_kv;
-  const int g = blockIdx.x % p.n_kv;
-  const int lane = threadIdx.x;
-  const int j = p.items[2 * item];
-  const int page = p.items[2 * item + 1];
-  // An item outside the record array (page >= max_pages) would write into the next
-  // row's records: it is skipped (the caller sizes max_pages for its longest row).
-  if (page < 0 || page >= p.max_pages) return;
+  constexpr int kPer = kAttnPage * D / kEl / 64;  // pieces of one page of V per lane
+  constexpr int kKey = D / kEl;                   // pieces of one K row
   const int slot = p.row_slot[j];
   const int visible = p.row_pos[j] + 1;
   const int p0 = page << kAttnPageShift;
-  const int n = min(visible - p0, kAttnPage);
-  __shared__ f32x4 q4[D];        // the four heads' query values, per dim
-  __shared__ f32x4 w4[kAttnPage];  // the four heads' weights, per position
-  __shared__ KvT vs[kAttnPage][D];
+  const int n = __builtin_amdgcn_readfirstlane(min(visible - p0, kAttnPage));
 
   // Positions past the row's last one are clamped to it (their values are never
   // used), so every load is unconditional and stays inside the row's own pages.
@@ -251,115 +329,458 @@ __global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int p
 #pragma unroll
     for (int c = 0; c < kKey; ++c) kr[c] = load16(key + kEl * c);
   }
-  const float* qrow = p.q + static_cast<int64_t>(j) * p.q_stride + static_cast<int64_t>(g * kHeadsPerGroup) * D;
-  for (int d = lane; d < D; d += 64)
-    q4[d] = f32x4{qrow[d], qrow[D + d], qrow[2 * D + d], qrow[3 * D + d]};
+  float qa[D / 16];
+  load_query<D>(p.q + static_cast<int64_t>(j) * p.q_stride + static_cast<int64_t>(g * kHeadsPerGroup) * D, lane, qa);
+  __builtin_amdgcn_sched_barrier(0);  // every load before the first use
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int P = k * 64 + lane;
-    *reinterpret_cast<u32x4*>(&vs[P / (D / kEl)][(P % (D / kEl)) * kEl]) = vr[k];
+    *reinterpret_cast<u32x4*>(&lds.vs[P / (D / kEl)][(P % (D / kEl)) * kEl]) = vr[k];
   }
-  __syncthreads();
-
-  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-#pragma unroll
-  for (int c = 0; c < kKey; ++c) {
-#pragma unroll
-    for (int e = 0; e < kEl; ++e) {
-      float k;
-      if constexpr (kEl == 8) k = f32_of(e & 1 ? kr[c][e >> 1] & 0xFFFF0000u : kr[c][e >> 1] << 16);
-      else k = f32_of(kr[c][e]);
-      const f32x4 qd = q4[kEl * c + e];
-      a0 = __builtin_fmaf(qd[0], k, a0);
-      a1 = __builtin_fmaf(qd[1], k, a1);
-      a2 = __builtin_fmaf(qd[2], k, a2);
-      a3 = __builtin_fmaf(qd[3], k, a3);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // keep each chunk's query reads next to their use
-  }
+  const f32x4 a = page_scores<D, KvT>(kr, qa);
   const float neg_inf = f32_of(0xFF800000u);
-  float sc[kHeadsPerGroup] = {a0 * p.scale, a1 * p.scale, a2 * p.scale, a3 * p.scale};
   f32x4 mx;
 #pragma unroll
   for (int h = 0; h < kHeadsPerGroup; ++h) {
-    if (lane >= n) sc[h] = neg_inf;
-    mx[h] = wave_max(sc[h]);
+    const float sc = lane < n ? a[h] * p.scale : neg_inf;
+    mx[h] = wave_max(sc);
+    if (lane < n) lds.wt[h * kAttnPage + lane] = det_exp(sc - mx[h]);
   }
-  if (lane < n) w4[lane] = f32x4{det_exp(sc[0] - mx[0]), det_exp(sc[1] - mx[1]), det_exp(sc[2] - mx[2]), det_exp(sc[3] - mx[3])};
-  __syncthreads();
+  wave_phase();
   float* rec = p.scratch + (static_cast<int64_t>(j * p.n_kv + g) * p.max_pages + page) * p.rec_floats;
-  float* v_out = rec + 8;
-  const float* wflat = reinterpret_cast<const float*>(w4);
-  float den = 0.0f;  // head (lane & 3)
+  f32x4 acc[(D + 63) / 64];
+  float den;
+  page_mix<D, KvT>(lds.wt, lds.vs, n, lane, acc, den);
 #pragma unroll
-  for (int it = 0; it < (D + 63) / 64; ++it) {
-    const int d = lane + 64 * it;
-    if (d >= D) continue;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-    for (int i = 0; i < n; ++i) {
-      float v;
-      if constexpr (kEl == 8) v = f32_of(static_cast<uint32_t>(vs[i][d]) << 16);
-      else v = vs[i][d];
-      const f32x4 wi = w4[i];
+  for (int t = 0; t < (D + 63) / 64; ++t)
 #pragma unroll
-      for (int h = 0; h < kHeadsPerGroup; ++h) acc[h] = __builtin_fmaf(wi[h], v, acc[h]);
-      if (it == 0) den = den + wflat[i * kHeadsPerGroup + (lane & 3)];
-    }
-#pragma unroll
-    for (int h = 0; h < kHeadsPerGroup; ++h) v_out[h * D + d] = acc[h];
-  }
+    for (int h = 0; h < kHeadsPerGroup; ++h)
+      if (lane + 64 * t < D) rec[8 + h * D + lane + 64 * t] = acc[t][h];
   if (lane < kHeadsPerGroup) {
     rec[lane] = mx[lane];
     rec[4 + lane] = den;
+  }
+  wave_phase();  // the next item's staging comes after this one's reads
+}
+
+// Tiles of kTileRows = 16 consecutive rows (k_attn_tile).
+constexpr int kTileRows = 16;
+
+// Lane l holds row l % 16: its slot, and its visible positions (0 past the last row).
+struct TileRow {
+  int slot, visible;
+};
+__device__ __forceinline__ TileRow tile_row(const StrideAttentionParams& p, int j0, int lane) {
+  const int nr = min(kTileRows, p.l.rows - j0), row = lane & (kTileRows - 1), j = j0 + min(row, nr - 1);
+  const int slot = p.row_slot[j], pos = p.row_pos[j];
+  return {slot, row < nr ? pos + 1 : 0};
+}
+
+// Do the rows lie in at most two sequences, at neighbouring positions? (Rows far apart
+// share few pages that are whole for all of them.)
+__device__ __forceinline__ bool tile_shared(TileRow tr) {
+  const int first = __builtin_amdgcn_readfirstlane(tr.slot);
+  int near = __builtin_amdgcn_readfirstlane(tr.visible);  // the position of this lane's sequence's first row
+  const uint64_t others = __ballot(tr.slot != first);
+  if (others != 0) {
+    const int r = __builtin_ctzll(others), second = __builtin_amdgcn_readlane(tr.slot, r);
+    if (__any(tr.slot != first && tr.slot != second)) return false;
+    if (tr.slot != first) near = __builtin_amdgcn_readlane(tr.visible, r);
+  }
+  return !__any(tr.visible > 0 && abs(tr.visible - near) > kAttnPage / 2);
+}
+
+// Does the item list hold every page of the tile's rows where the pages of the rows
+// before them end (as the engine's list does, src/engine.cpp:93-103)?
+__device__ __forceinline__ bool tile_listed(const StrideAttentionParams& p, int j0, int lane, TileRow tr) {
+  const int pages = (tr.visible + kAttnPage - 1) >> kAttnPageShift;
+  if (__any(pages > p.max_pages)) return false;
+  int lo = 0;  // items of the rows before the tile
+#pragma unroll 16
+  for (int r = lane; r < j0; r += 64) lo += (p.row_pos[r] >> kAttnPageShift) + 1;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) lo += __shfl_xor(lo, off);
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  int end[kTileRows];  // items of the tile's rows up to each one
+  int total = 0;
+#pragma unroll
+  for (int r = 0; r < kTileRows; ++r) end[r] = total += __builtin_amdgcn_readlane(pages, r);
+  if (total > p.item_count - lo) return false;
+  bool ok = true;
+#pragma unroll 4
+  for (int u = lane; u < total; u += 64) {
+    int r = 0, c = u;  // item u of the tile: row r, page c
+#pragma unroll
+    for (int e = 0; e + 1 < kTileRows; ++e)
+      if (u >= end[e]) {
+        r = e + 1;
+        c = u - end[e];
+      }
+    ok = ok & (p.items[2 * (lo + u)] == j0 + r) & (p.items[2 * (lo + u) + 1] == c);
+  }
+  return __all(ok);
+}
+
+// A tile's pages for one KV group: workgroup (tile, group, walker) takes pages walker,
+// walker + walkers, ... of it and stores the records of page_item. Rows of one sequence
+// share the pages that they read, and there the fmaf chains run as fp32 MFMAs (v_mfma_f32_16x16x4_f32 adds its four products in order, one rounding
+// each: a chain of fmaf, bit for bit), K and V of a page being staged once, widened, for
+// the sixteen rows. A wave holds four rows x four heads as the 16 columns i = 4 * row +
+// head of the score tile (its rows: 16 positions; lane l holds column l % 16). Position
+// 4v + a of a tile is its row 4a + v, so a lane's score register v of quarter a = l / 16
+// is the mix's left operand of step v as it stands: the weights never leave their
+// registers. They are also multiplied by ones (one more column tile of the mix), which
+// adds the denominators in order. Positions past a row's last one must not enter its
+// sums at all (a product with a zero weight could turn -0 into +0, or infinity into
+// NaN): a page that is not whole for all of the wave's rows takes whole steps as MFMAs
+// and its last few positions as fmaf under the row's own bound. Tiles whose rows
+// share nothing (decode rows) are left to k_attn_page; a tile whose pages are not all
+// listed is taken item by item.
+//
+// Bound by the fp32 units, which the MFMAs (144 of 32 cycles a wave and page) and vector
+// instructions (490 of 4 cycles) take in turn: 82 % of them busy at 2048 rows of one
+// prompt, 8 groups, head_dim 64: 212 us, against 507 us a wave per item on the vector
+// pipe alone.
+template <int D, class KvT>
+__global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_attn_tile(StrideAttentionParams p, int page_shift,
+                                                                                     int walkers) {
+  constexpr int kEl = 16 / static_cast<int>(sizeof(KvT));  // KV elements per 16-byte piece
+  constexpr int kRow = D / kEl;                    // pieces of one K or V row
+  constexpr int kPer = kAttnPage * kRow / 256;     // pieces of one page per thread
+  constexpr int S4 = D / 4;                        // score steps
+  constexpr int KS = D + 4;                        // K row stride in LDS (conflict-free column reads)
+  constexpr int NDT = D / 16;                      // output column tiles
+  constexpr int VW = D >= 64 ? 4 : 2;              // dims a lane reads of a V row at a time
+  typedef float Word __attribute__((ext_vector_type(VW), aligned(4)));
+  struct Tile {
+    float ks[kAttnPage * KS];  // K: position, then dims 4s + a at a * S4 + s
+    float vs[kAttnPage * D];
+    float wb[4][16 * 16];      // a wave's weights of 16 positions
+  };
+  constexpr int kItemWaves = 4 * sizeof(PageLds<D, KvT>) <= sizeof(Tile) + 8192 ? 4 : 2;  // waves taking single items
+  union Lds {
+    Tile t;
+    PageLds<D, KvT> item[kItemWaves];
+  };
+  __shared__ __align__(16) unsigned char lds_bytes[sizeof(Lds)];
+  Lds& lds = *reinterpret_cast<Lds*>(lds_bytes);
+  auto& ks = lds.t.ks;
+  auto& vs = lds.t.vs;
+  auto& wb = lds.t.wb;
+  extern __shared__ uint32_t listed[];  // [kTileRows][words] bits, lists that are not the engine's
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int per_tile = p.n_kv * walkers;
+  const int blocks = (p.l.rows + kTileRows - 1) / kTileRows;
+  // Later rows of a prompt read more pages: their workgroups start first.
+  const int j0 = (blocks - 1 - static_cast<int>(blockIdx.x) / per_tile) * kTileRows;
+  const int g = blockIdx.x % p.n_kv, walker = static_cast<int>(blockIdx.x) % per_tile / p.n_kv;
+  const int rows4 = wave * 4;
+  const TileRow tr = tile_row(p, j0, lane);
+  if (!tile_shared(tr)) return;  // k_attn_page takes its items
+  const bool whole = tile_listed(p, j0, lane, tr);
+  if (whole && !__any(walker << kAttnPageShift < tr.visible)) return;
+  if (!whole) {
+    const int nr = min(kTileRows, p.l.rows - j0), words = (p.max_pages + 31) / 32;
+    for (int u = tid; u < kTileRows * words; u += 256) listed[u] = 0u;
+    __syncthreads();
+    for (int u = tid; u < p.item_count; u += 256) {
+      const int r = p.items[2 * u] - j0, c = p.items[2 * u + 1];
+      if (r >= 0 && r < nr && c >= 0 && c < p.max_pages) atomicOr(&listed[r * words + (c >> 5)], 1u << (c & 31));
+    }
+    __syncthreads();
+    if (wave >= kItemWaves) return;
+    for (int c = walker; c < p.max_pages; c += walkers)
+      for (int r = wave; r < nr; r += kItemWaves)
+        if ((listed[r * words + (c >> 5)] >> (c & 31)) & 1u)
+          page_item<D, KvT>(p, page_shift, j0 + r, c, g, lane, lds.item[wave]);
+    return;
+  }
+  const float neg_inf = f32_of(0xFF800000u);
+  const int i = lane & 15, q = lane >> 4;
+
+  // The rows of one sequence at a time (usually all sixteen).
+  int slot = __builtin_amdgcn_readfirstlane(tr.slot);
+  for (;;) {
+    const int mine = tr.slot == slot ? tr.visible : 0;  // 0 for rows that are not the sequence's
+    int last = 0;  // last position any of the sequence's rows sees
+#pragma unroll
+    for (int r = 0; r < kTileRows; ++r) last = max(last, __builtin_amdgcn_readlane(mine, r));
+    --last;
+    const int pages = (last >> kAttnPageShift) + 1;
+    // Visible positions of the wave's rows, the least (of the sequence's) and the most.
+    const int n0 = __builtin_amdgcn_readlane(mine, rows4), n1 = __builtin_amdgcn_readlane(mine, rows4 + 1);
+    const int n2 = __builtin_amdgcn_readlane(mine, rows4 + 2), n3 = __builtin_amdgcn_readlane(mine, rows4 + 3);
+    const int far = p.max_pages * kAttnPage;
+    const int lo = min(min(n0 > 0 ? n0 : far, n1 > 0 ? n1 : far), min(n2 > 0 ? n2 : far, n3 > 0 ? n3 : far));
+    const int hi = max(max(n0, n1), max(n2, n3));
+    // This lane's row as a score column (row i / 4) and as an output row (row q).
+    const int vis_i = (i >> 2) < 2 ? ((i >> 2) == 0 ? n0 : n1) : ((i >> 2) == 2 ? n2 : n3);
+    const int vis_d = q < 2 ? (q == 0 ? n0 : n1) : (q == 2 ? n2 : n3);
+    float qv[S4];
+    {
+      const int j = min(j0 + rows4 + (i >> 2), p.l.rows - 1);
+      const float* src = p.q + static_cast<int64_t>(j) * p.q_stride + static_cast<int64_t>(g * kHeadsPerGroup + (i & 3)) * D + q;
+#pragma unroll
+      for (int e = 0; e < S4; ++e) qv[e] = src[4 * e];
+    }
+
+    // Staging: piece P = k * 256 + tid of a page is piece P % kRow of position P / kRow;
+    // the page numbers of the page after next, and the pieces of the next page, are in
+    // flight while a page is summed. Positions past `last` are loaded from it.
+    int blk[kPer];
+    u32x4 kr[kPer], vr[kPer];
+    const KvT* base = static_cast<const KvT*>(p.kv.arena) + p.layer * p.kv.layer_elems + g * p.kv.group_elems + (tid % kRow) * kEl;
+    const int32_t* table = p.kv.table + static_cast<int64_t>(slot) * p.kv.max_blocks;
+    auto pos_of = [&](int page, int k) { return min((page << kAttnPageShift) + (k * 256 + tid) / kRow, last); };
+    auto load_blk = [&](int page) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) blk[k] = table[pos_of(page, k) >> page_shift];
+    };
+    auto fetch = [&](int page) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        const KvT* at = base + blk[k] * p.kv.block_elems + (pos_of(page, k) & ((1 << page_shift) - 1)) * D;
+        kr[k] = load16(at);
+        vr[k] = load16(at + p.kv.which_elems);
+      }
+      load_blk(page + walkers);
+    };
+    auto widen = [&](const u32x4& v, int e) {
+      if constexpr (kEl == 8) return f32_of(e & 1 ? v[e >> 1] & 0xFFFF0000u : v[e >> 1] << 16);
+      else return f32_of(v[e]);
+    };
+    load_blk(walker);
+    fetch(walker);
+    for (int c = walker; c < pages; c += walkers) {
+      const int p0 = c << kAttnPageShift;
+      lds_barrier();  // the last page has been read
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        const int pos = (k * 256 + tid) / kRow, d = (tid % kRow) * kEl;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          float* dst = &ks[pos * KS + a * S4 + d / 4];
+          if constexpr (kEl == 8) *reinterpret_cast<f32x2*>(dst) = f32x2{widen(kr[k], a), widen(kr[k], 4 + a)};
+          else *dst = widen(kr[k], a);
+        }
+        f32x4* dst = reinterpret_cast<f32x4*>(&vs[pos * D + d]);
+#pragma unroll
+        for (int e = 0; e < kEl / 4; ++e)
+          dst[e] = f32x4{widen(vr[k], 4 * e), widen(vr[k], 4 * e + 1), widen(vr[k], 4 * e + 2), widen(vr[k], 4 * e + 3)};
+      }
+      lds_barrier();
+      if (c + walkers < pages) fetch(c + walkers);
+      if (p0 >= hi) continue;
+      // Scores of positions 16t + 4v + q for column i; past the row's last one -inf.
+      f32x4 w[4];
+      const f32x4* src = reinterpret_cast<const f32x4*>(&ks[(4 * (i & 3) + (i >> 2)) * KS + q * S4]);
+      unroll<S4 / 4>([&](auto ee) {
+        constexpr int e = decltype(ee)::value;
+        f32x4 k4[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) k4[t] = src[t * 4 * KS + e];
+        unroll<16>([&](auto xx) {
+          constexpr int x = decltype(xx)::value / 4, t = decltype(xx)::value % 4;
+          const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+          w[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[t][x], qv[4 * e + x], e == 0 && x == 0 ? zero : w[t], 0, 0, 0);
+        });
+      });
+      const bool partial = p0 + kAttnPage > lo;
+      const int n_i = vis_i - p0;
+      float mx = neg_inf;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w[t] = w[t] * p.scale;
+      if (partial) {
+        unroll<16>([&](auto ee) {
+          constexpr int t = decltype(ee)::value / 4, v = decltype(ee)::value % 4;
+          if (16 * t + 4 * v + q >= n_i) w[t][v] = neg_inf;
+        });
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) mx = fmaxf(mx, w[t][v]);
+      {  // over the column's four quarters
+        const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+        const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+      }
+      unroll<16>([&](auto ee) {
+        constexpr int t = decltype(ee)::value / 4, v = decltype(ee)::value % 4;
+        w[t][v] = det_exp(w[t][v] - mx);
+      });
+      f32x4 mix[NDT], dn = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int t = 0; t < NDT; ++t) mix[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      // Output column of tile t: dim 64 * (t / 4) + 4 * i + t % 4 (D = 32: 2 * i + t).
+      auto v_row = [&](int pos, float (&vv)[NDT]) {
+#pragma unroll
+        for (int hh = 0; hh < NDT / VW; ++hh) {
+          const Word x = *reinterpret_cast<const Word*>(&vs[pos * D + 64 * hh + VW * i]);
+#pragma unroll
+          for (int e = 0; e < VW; ++e) vv[VW * hh + e] = x[e];
+        }
+      };
+      if (!partial) {
+        unroll<16>([&](auto ee) __attribute__((always_inline)) {
+          constexpr int e = decltype(ee)::value;
+          float vv[NDT];
+          v_row(4 * e + q, vv);
+          const float a = w[e / 4][e % 4];
+          dn = __builtin_amdgcn_mfma_f32_16x16x4f32(a, 1.0f, dn, 0, 0, 0);
+          unroll<NDT>([&](auto tt) {
+            constexpr int t = decltype(tt)::value;
+            mix[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vv[t], mix[t], 0, 0, 0);
+          });
+        });
+      } else {
+        // Steps that not all of the wave's rows see whole multiply -0 by 1: a sum plus -0
+        // is that sum, whatever it is. (Branches around them would expose every LDS read.)
+        const int whole_steps = min(max(lo - p0, 0), kAttnPage) / 4;
+        unroll<16>([&](auto ee) __attribute__((always_inline)) {
+          constexpr int e = decltype(ee)::value;
+          const bool live = e < whole_steps;
+          float vv[NDT];
+          v_row(4 * e + q, vv);
+          const float a = live ? w[e / 4][e % 4] : -0.0f;
+          dn = __builtin_amdgcn_mfma_f32_16x16x4f32(a, 1.0f, dn, 0, 0, 0);
+          unroll<NDT>([&](auto tt) {
+            constexpr int t = decltype(tt)::value;
+            mix[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, live ? vv[t] : 1.0f, mix[t], 0, 0, 0);
+          });
+        });
+        const int n_d = vis_d - p0, end = min(hi - p0, kAttnPage);
+        for (int c0 = 4 * whole_steps; c0 < end; c0 += 16) {  // usually once
+          __builtin_amdgcn_wave_barrier();
+          unroll<16>([&](auto ee) __attribute__((always_inline)) {
+            constexpr int t = decltype(ee)::value / 4, v = decltype(ee)::value % 4;
+            const int at = 16 * t + 4 * v + q - c0;
+            if (at >= 0 && at < 16) wb[wave][at * 16 + i] = w[t][v];
+          });
+          __builtin_amdgcn_wave_barrier();
+          for (int pos = c0; pos < min(c0 + 16, end); pos += 4) {
+            f32x4 wv[4];
+            float vv[4][NDT];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              wv[e] = *reinterpret_cast<const f32x4*>(&wb[wave][(pos - c0 + e) * 16 + 4 * q]);
+              v_row(pos + e, vv[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (pos + e < n_d) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                  dn[v] = dn[v] + wv[e][v];
+#pragma unroll
+                  for (int u = 0; u < NDT; ++u) mix[u][v] = __builtin_fmaf(wv[e][v], vv[e][u], mix[u][v]);
+                }
+              }
+          }
+        }
+      }
+      auto record = [&](int row) {
+        return p.scratch + ((static_cast<int64_t>(j0 + rows4 + row) * p.n_kv + g) * p.max_pages + c) * p.rec_floats;
+      };
+      if (q == 0 && n_i > 0) record(i >> 2)[i & 3] = mx;
+      if (p0 < vis_d) {
+        float* rec = record(q);
+        if (i == 0) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) rec[4 + v] = dn[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int hh = 0; hh < NDT / VW; ++hh) {
+            Word x;
+#pragma unroll
+            for (int e = 0; e < VW; ++e) x[e] = mix[VW * hh + e][v];
+            *reinterpret_cast<Word*>(&rec[8 + v * D + 64 * hh + VW * i]) = x;
+          }
+      }
+    }
+    // the other sequence's rows, if the first row's have just been done
+    const uint64_t others = __ballot(tr.slot != __builtin_amdgcn_readfirstlane(tr.slot));
+    if (others == 0 || slot != __builtin_amdgcn_readfirstlane(tr.slot)) break;
+    slot = __builtin_amdgcn_readlane(tr.slot, __builtin_ctzll(others));
+  }
+}
+
+// Items one by one: a wave takes `per_wg` (at most 64) consecutive items of one KV
+// group. TILED: the items of tiles that k_attn_tile takes are skipped. An item outside
+// the record array (page >= max_pages) would write into the next row's records: it is
+// skipped (the caller sizes max_pages for its longest row).
+template <int D, class KvT, bool TILED>
+__global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int page_shift, int per_wg) {
+  __shared__ PageLds<D, KvT> lds;
+  const int g = blockIdx.x % p.n_kv, lane = threadIdx.x;
+  if constexpr (!TILED) {  // per_wg = 1
+    const int one = static_cast<int>(blockIdx.x) / p.n_kv;
+    const int j = p.items[2 * one], page = p.items[2 * one + 1];
+    if (page >= 0 && page < p.max_pages) page_item<D, KvT>(p, page_shift, j, page, g, lane, lds);
+    return;
+  }
+  const int item = static_cast<int>(blockIdx.x) / p.n_kv * per_wg + lane;  // this lane's
+  int row = 0, page = -1;
+  if (lane < per_wg && item < p.item_count) {
+    row = p.items[2 * item];
+    page = p.items[2 * item + 1];
+  }
+  uint64_t todo = __ballot(page >= 0 && page < p.max_pages);
+  for (uint64_t left = todo; left != 0;) {
+    const int j0 = __builtin_amdgcn_readlane(row, __builtin_ctzll(left)) & ~(kTileRows - 1);
+    const uint64_t of_tile = __ballot((row & ~(kTileRows - 1)) == j0);
+    if (tile_shared(tile_row(p, j0, lane))) todo &= ~of_tile;
+    left &= ~of_tile;
+  }
+  for (; todo != 0; todo &= todo - 1) {
+    const int n = __builtin_ctzll(todo);
+    page_item<D, KvT>(p, page_shift, __builtin_amdgcn_readlane(row, n), __builtin_amdgcn_readlane(page, n), g, lane, lds);
   }
 }
 
 // Ascending-page combine of one row's records for one KV group, written as bf16
 // x tiles (src/kernel_common.h:252-309, writer src/kernels_tc.cu:658-666) or,
 // for the exact path, as fp32 dim-major out[idx * stride + row] (LaneWriter,
-// src/kernels.cu:287-291). All
-// of the row's records come into LDS in one coalesced pass; threads 0..3 derive
-// each head's page factors and denominator (pages in order); thread (h, d) then
-// folds the weighted values of head h, dim d over the pages in order.
+// src/kernels.cu:287-291). Bound by reading the records once. Wave h derives head h's
+// page factors, a page per lane; then thread (h, d) folds the weighted values of head h,
+// dim d over the pages in order, straight from memory (a page's are 1 KiB at head_dim
+// 64), with the denominator beside them. 2048 rows of up to 32 pages, 8 groups: 181 us
+// when one thread per head walked the pages and all records went through LDS.
 template <int D, bool kExact>
 __global__ __launch_bounds__(256) void k_attn_combine(StrideAttentionParams p) {
-  extern __shared__ float recs[];  // [pages][rec_floats], then f[4][pages]
-  __shared__ float den[kHeadsPerGroup];
+  extern __shared__ f32x2 fd[];  // [4][pages]: page factor, page denominator
   const int j = blockIdx.x / p.n_kv;
   const int g = blockIdx.x % p.n_kv;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int pages = min((p.row_pos[j] >> kAttnPageShift) + 1, p.max_pages);  // row_pos < 64 * max_pages
-  const int rf = p.rec_floats;
-  const float* src = p.scratch + static_cast<int64_t>(j * p.n_kv + g) * p.max_pages * rf;
-  for (int i = t; i < pages * rf; i += 256) recs[i] = src[i];
-  float* f = recs + pages * rf;
-  __syncthreads();
-  if (t < kHeadsPerGroup) {
+  const int64_t rf = p.rec_floats;
+  const float* recs = p.scratch + static_cast<int64_t>(j * p.n_kv + g) * p.max_pages * rf;
+  {
     float m = f32_of(0xFF800000u);
-    for (int c = 0; c < pages; ++c) {
-      const float mc = recs[c * rf + t];
-      if (mc > m) m = mc;
-    }
-    float d = 0.0f;
-    for (int c = 0; c < pages; ++c) {
-      const float e = det_exp(recs[c * rf + t] - m);
-      f[t * pages + c] = e;
-      d = __builtin_fmaf(e, recs[c * rf + 4 + t], d);
-    }
-    den[t] = d;
+    for (int c = lane; c < pages; c += 64) m = pick_gt(recs[c * rf + wave], m);
+    m = wave_max(m);
+    for (int c = lane; c < pages; c += 64) fd[wave * pages + c] = f32x2{det_exp(recs[c * rf + wave] - m), recs[c * rf + 4 + wave]};
   }
   __syncthreads();
   const int col_tiles = p.out_cols >> 4;
   uint16_t* out = static_cast<uint16_t*>(p.out);
   const int64_t lane0 = static_cast<int64_t>(j >> 4) * col_tiles * kTileElems + (j & 15) * 16;
-  for (int hd = t; hd < p.n_q * D; hd += 256) {
+  for (int hd = t; hd < kHeadsPerGroup * D; hd += 256) {
     const int qh = hd / D, d = hd % D;
-    float acc = 0.0f;
-    for (int c = 0; c < pages; ++c) acc = __builtin_fmaf(f[qh * pages + c], recs[c * rf + 8 + qh * D + d], acc);
-    const int idx = (g * p.n_q + qh) * D + d;
-    if constexpr (kExact) static_cast<float*>(p.out)[static_cast<int64_t>(idx) * p.l.stride + j] = acc / den[qh];
-    else out[lane0 + static_cast<int64_t>(idx >> 4) * kTileElems + (idx & 15)] = static_cast<uint16_t>(bf16_rne(acc / den[qh]));
+    const f32x2* f = fd + qh * pages;
+    float acc = 0.0f, dn = 0.0f;
+#pragma unroll 8
+    for (int c = 0; c < pages; ++c) {
+      const f32x2 e = f[c];
+      dn = __builtin_fmaf(e[0], e[1], dn);
+      acc = __builtin_fmaf(e[0], recs[c * rf + 8 + hd], acc);
+    }
+    const int idx = (g * kHeadsPerGroup + qh) * D + d;
+    if constexpr (kExact) static_cast<float*>(p.out)[static_cast<int64_t>(idx) * p.l.stride + j] = acc / dn;
+    else out[lane0 + static_cast<int64_t>(idx >> 4) * kTileElems + (idx & 15)] = static_cast<uint16_t>(bf16_rne(acc / dn));
   }
 }
 
@@ -392,7 +813,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_fused(StrideAttentionParams p
   constexpr int kKey = D / kEl;                 // 16-byte pieces of one K row
   constexpr int RF = 8 + kHeadsPerGroup * D;    // record floats
   extern __shared__ float recs[];  // [max_pages][RF], f[4][max_pages], then the row's KV page numbers
-  __shared__ f32x4 w4[NWV][kAttnPage];
+  __shared__ __align__(16) float wt[NWV][kHeadsPerGroup * kAttnPage];  // weights [head][position]
   __shared__ KvT vs[NWV][kAttnPage][D];
   __shared__ uint32_t listed[LIST ? kListMaxPages / 32 : 1];
   __shared__ int part[NWV];
@@ -417,10 +838,8 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_fused(StrideAttentionParams p
   };
   __syncthreads();
   const float* qrow = p.q + static_cast<int64_t>(j) * p.q_stride + static_cast<int64_t>(g * kHeadsPerGroup) * D;
-  // The query row is the same for every lane: read through the scalar cache into
-  // SGPRs, so the scores take their query operands without LDS reads.
-  typedef const __attribute__((address_space(4))) float ConstF;
-  ConstF* cq = (ConstF*)(qrow);
+  float qa[D / 16];
+  load_query<D>(qrow, lane, qa);
   const float neg_inf = f32_of(0xFF800000u);
   const int rounds = (pages + NWV - 1) / NWV;  // the same for every wave: barriers stay uniform
   // K and V of the wave's next page are loaded into registers one round ahead:
@@ -488,27 +907,9 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_fused(StrideAttentionParams p
     f32x4 mx = {0.f, 0.f, 0.f, 0.f};
     float sc[kHeadsPerGroup] = {0.f, 0.f, 0.f, 0.f};
     if (active) {
-      float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+      const f32x4 a = page_scores<D, KvT>(kr, qa);
 #pragma unroll
-      for (int c = 0; c < kKey; ++c) {
-#pragma unroll
-        for (int e = 0; e < kEl; ++e) {
-          float k;
-          if constexpr (kEl == 8) k = f32_of(e & 1 ? kr[c][e >> 1] & 0xFFFF0000u : kr[c][e >> 1] << 16);
-          else k = f32_of(kr[c][e]);
-          const int d = kEl * c + e;
-          const f32x4 qd = f32x4{cq[d], cq[D + d], cq[2 * D + d], cq[3 * D + d]};
-          a0 = __builtin_fmaf(qd[0], k, a0);
-          a1 = __builtin_fmaf(qd[1], k, a1);
-          a2 = __builtin_fmaf(qd[2], k, a2);
-          a3 = __builtin_fmaf(qd[3], k, a3);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      sc[0] = a0 * p.scale;
-      sc[1] = a1 * p.scale;
-      sc[2] = a2 * p.scale;
-      sc[3] = a3 * p.scale;
+      for (int h = 0; h < kHeadsPerGroup; ++h) sc[h] = a[h] * p.scale;
     }
     if (page + NWV < pages) fetch(page + NWV);  // registers are free again
     if (active) {
@@ -516,33 +917,20 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_fused(StrideAttentionParams p
       for (int h = 0; h < kHeadsPerGroup; ++h) {
         if (lane >= n) sc[h] = neg_inf;
         mx[h] = wave_max(sc[h]);
+        if (lane < n) wt[wave][h * kAttnPage + lane] = det_exp(sc[h] - mx[h]);
       }
-      if (lane < n)
-        w4[wave][lane] = f32x4{det_exp(sc[0] - mx[0]), det_exp(sc[1] - mx[1]), det_exp(sc[2] - mx[2]), det_exp(sc[3] - mx[3])};
     }
     __syncthreads();  // this wave's weights
     if (active) {
       float* rec = recs + page * RF;
-      const float* wflat = reinterpret_cast<const float*>(w4[wave]);
-      float dn = 0.0f;  // head (lane & 3)
+      f32x4 acc[(D + 63) / 64];
+      float dn;
+      page_mix<D, KvT>(wt[wave], vs[wave], __builtin_amdgcn_readfirstlane(n), lane, acc, dn);
 #pragma unroll
-      for (int itd = 0; itd < (D + 63) / 64; ++itd) {
-        const int d = lane + 64 * itd;
-        if (d >= D) continue;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 8
-        for (int i = 0; i < n; ++i) {
-          float v;
-          if constexpr (kEl == 8) v = f32_of(static_cast<uint32_t>(vs[wave][i][d]) << 16);
-          else v = vs[wave][i][d];
-          const f32x4 wi = w4[wave][i];
+      for (int t = 0; t < (D + 63) / 64; ++t)
 #pragma unroll
-          for (int h = 0; h < kHeadsPerGroup; ++h) acc[h] = __builtin_fmaf(wi[h], v, acc[h]);
-          if (itd == 0) dn = dn + wflat[i * kHeadsPerGroup + (lane & 3)];
-        }
-#pragma unroll
-        for (int h = 0; h < kHeadsPerGroup; ++h) rec[8 + h * D + d] = acc[h];
-      }
+        for (int h = 0; h < kHeadsPerGroup; ++h)
+          if (lane + 64 * t < D) rec[8 + h * D + lane + 64 * t] = acc[t][h];
       if (lane < kHeadsPerGroup) {
         rec[lane] = mx[lane];
         rec[4 + lane] = dn;
@@ -632,23 +1020,9 @@ static_assert(offsetof(StrideAttentionParams, kv) == 48 && sizeof(StrideAttentio
 
 static int launched(const char* what);
 
-// The combine keeps a row's records in LDS; past the default 64 KiB of dynamic
-// LDS (long contexts at head_dim 128) the kernel's limit is raised once.
-// (The kernel's own static LDS shares the 160 KiB, hence the margin.)
+// LDS that the records of a row may take (the kernel's own static LDS shares the 160
+// KiB, hence the margin).
 constexpr size_t kCombineLdsMax = 159 * 1024;
-
-template <int D, bool kExact>
-static int combine(dim3 grid, size_t lds, hipStream_t st, const StrideAttentionParams& p) {
-  static size_t raised = 64 * 1024;
-  if (lds > raised) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_combine<D, kExact>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    if (e != hipSuccess) return fail(static_cast<int>(e), std::string("tc_attention: raising the LDS limit failed: ") + hipGetErrorString(e));
-    raised = lds;
-  }
-  hipLaunchKernelGGL((k_attn_combine<D, kExact>), grid, dim3(256), lds, st, p);
-  return launched("attention (combine)");
-}
 
 // One-kernel attention; its static LDS (staging for up to four waves) and the
 // row's records share the 160 KiB.
@@ -694,6 +1068,41 @@ static bool fused_fits(size_t lds) {
 // for up to this many rows: each workgroup sums the page counts of the rows
 // before its own to find its stretch of the list, which grows with the row count.
 constexpr int kListFusedMaxRows = 512;
+
+// Page sums and combine in launches of their own.
+template <int D, class KvT, bool kExact>
+static int paged(hipStream_t st, const StrideAttentionParams& p, int page_shift) {
+  // Tiles for 128 to 8192 rows (a smaller batch that comes here, contexts beyond the
+  // one-kernel form's LDS, may as well be decode rows, and each tile adds up the pages of
+  // all rows before it) and long lists: finding out what is whose costs two to three
+  // launches' latency, which 32768 items and groups are worth (whole attention, tiles
+  // against items: 18.5 k 38 against 45 us, 26.6 k 62 / 69, 41.6 k 77 / 100, but 19.7 k, four prompts of
+  // 250 rows between other kernels, 60 / 57, and 28.8 k of 600 decode rows, which take
+  // both ways, 81 / 70; 82 k 144, 270 k 273 us, against 203 and 695 before there were tiles).
+  const int64_t waves = static_cast<int64_t>(p.item_count) * p.n_kv;
+  if (waves > 32768 && p.l.rows >= 128 && p.l.rows <= 8192) {
+    // Walkers: as many workgroups as the chip holds at once, about four to a CU (1000
+    // rows in four prompts, 504 tiles and groups: 36 us with two walkers, 39 with one,
+    // 45 with four, which look at the list for one page each).
+    const int tiles = (p.l.rows + kTileRows - 1) / kTileRows * p.n_kv;
+    const int walkers = std::max(1, std::min(p.max_pages, 1024 / tiles));
+    const size_t bits = static_cast<size_t>(kTileRows) * ((p.max_pages + 31) / 32) * sizeof(uint32_t);
+    hipLaunchKernelGGL((k_attn_tile<D, KvT>), dim3(tiles * walkers), dim3(256), bits, st, p, page_shift, walkers);
+    if (int rc = launched("attention (tiles)")) return rc;
+    // Where the tiles take everything the waves below only find that out: several items
+    // each, but waves enough for decode rows' items.
+    const int per_wg = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(64, waves / 16384)));
+    const dim3 grid((p.item_count + per_wg - 1) / per_wg * p.n_kv);
+    hipLaunchKernelGGL((k_attn_page<D, KvT, true>), grid, dim3(64), 0, st, p, page_shift, per_wg);
+    if (int rc = launched("attention (pages)")) return rc;
+  } else if (p.item_count > 0) {
+    hipLaunchKernelGGL((k_attn_page<D, KvT, false>), dim3(p.item_count * p.n_kv), dim3(64), 0, st, p, page_shift, 1);
+    if (int rc = launched("attention (pages)")) return rc;
+  }
+  const size_t lds = static_cast<size_t>(p.max_pages) * kHeadsPerGroup * sizeof(f32x2);
+  hipLaunchKernelGGL((k_attn_combine<D, kExact>), dim3(p.l.rows * p.n_kv), dim3(256), lds, st, p);
+  return launched("attention (combine)");
+}
 
 static int launched(const char* what) {
   const hipError_t e = hipGetLastError();
@@ -785,18 +1194,9 @@ static int attention(const StrideAttentionParams* p, void* stream, const char* n
       return fused<128, true, KvT, kExact>(grid, lds, st, *p, page_shift);
     }
   }
-  if (p->item_count > 0) {
-    const dim3 grid(p->item_count * p->n_kv);
-    if (D == 32) hipLaunchKernelGGL((k_attn_page<32, KvT>), grid, dim3(64), 0, st, *p, page_shift);
-    else if (D == 64) hipLaunchKernelGGL((k_attn_page<64, KvT>), grid, dim3(64), 0, st, *p, page_shift);
-    else hipLaunchKernelGGL((k_attn_page<128, KvT>), grid, dim3(64), 0, st, *p, page_shift);
-    if (int rc = launched("attention (pages)")) return rc;
-  }
-  const size_t lds = static_cast<size_t>(p->max_pages) * (p->rec_floats + kHeadsPerGroup) * sizeof(float);
-  const dim3 cgrid(p->l.rows * p->n_kv);
-  if (D == 32) return combine<32, kExact>(cgrid, lds, st, *p);
-  if (D == 64) return combine<64, kExact>(cgrid, lds, st, *p);
-  return combine<128, kExact>(cgrid, lds, st, *p);
+  if (D == 32) return paged<32, KvT, kExact>(st, *p, page_shift);
+  if (D == 64) return paged<64, KvT, kExact>(st, *p, page_shift);
+  return paged<128, KvT, kExact>(st, *p, page_shift);
 }
 
 extern "C" int stride_tc_attention(const StrideAttentionParams* p, void* stream) {

@@ -134,6 +134,14 @@ __device__ __forceinline__ f32x16 block_of_tiles(const f32x4 (&t)[2][2], int lan
   return v;
 }
 
+// Workgroup barrier that orders LDS accesses only (loads from memory stay in flight,
+// which __syncthreads would wait for).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 __device__ __forceinline__ float f32_of(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ uint32_t u32_of(float f) { return __float_as_uint(f); }
 
@@ -147,9 +155,9 @@ __device__ __forceinline__ uint32_t bf16_rne(float f) {
 // Deterministic exp (src/numerics.h:16-30): k = floor(x*log2e + 1/2), two-part
 // Cody-Waite ln2 reduction, degree-6 Cephes polynomial by FMA, exponent scale.
 // Only correctly rounded operations (fma, floor, add) so the bits are fixed.
+// The range ends are selects, not returns: lanes differ in them, and several calls in a
+// row interleave only without branches.
 __device__ __forceinline__ float det_exp(float x) {
-  if (x < -87.0f) return 0.0f;
-  if (x > 88.0f) return f32_of(0x7F800000u);
   const float kf = floorf(fmaf(x, 1.44269504088896341f, 0.5f));
   float r = fmaf(-kf, 0.693359375f, x);
   r = fmaf(-kf, -2.12194440e-4f, r);
@@ -160,7 +168,9 @@ __device__ __forceinline__ float det_exp(float x) {
   p = fmaf(p, r, 1.6666665459e-1f);
   p = fmaf(p, r, 5.0000001201e-1f);
   const float y = fmaf(fmaf(p, r, 1.0f), r, 1.0f);
-  return f32_of(u32_of(y) + (static_cast<uint32_t>(static_cast<int32_t>(kf)) << 23));
+  float v = f32_of(u32_of(y) + (static_cast<uint32_t>(__float2int_rz(kf)) << 23));
+  asm("" : "+v"(v));  // no instruction: keeps the polynomial out of a branch on x
+  return x < -87.0f ? 0.0f : (x > 88.0f ? f32_of(0x7F800000u) : v);
 }
 
 // x * sigmoid(x) as x / (1 + exp(-x)); the division is IEEE (hipcc's default
