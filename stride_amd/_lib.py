@@ -276,6 +276,26 @@ def load(path: str = LIB_PATH) -> C.CDLL:
     return lib
 
 
+_packed = None
+
+
+def packed() -> C.CDLL:
+    """The library with entry points that take their parameter block as packed bytes
+    (struct.pack in the layouts above). Filling a ctypes Structure field by field took
+    4-11 us of Python per call, more than a small kernel runs; packing takes about 1."""
+    global _packed
+    if _packed is None:
+        load()
+        lib = C.CDLL(LIB_PATH)  # the same library: function objects with other argument types
+        for name, ints in (("embed", 0), ("norm", 1), ("qkv", 0), ("attention", 0), ("gemm_residual", 2), ("mlp13", 2),
+                           ("lm_greedy", 2), ("lm_full", 1)):
+            fn = getattr(lib, "stride_tc_" + name)
+            fn.argtypes = [C.c_char_p] + [C.c_int] * ints + [C.c_void_p]
+            fn.restype = C.c_int
+        _packed = lib
+    return _packed
+
+
 def check(rc: int) -> None:
     if rc != 0:
         msg = load().stride_tc_last_error().decode()

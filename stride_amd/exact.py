@@ -34,7 +34,8 @@ except ImportError:  # layout helpers still work on numpy arrays
 def _call(name: str, p, J=None) -> None:
     fn = getattr(_lib.load(), name)
     rc = fn(C.byref(p), tc.kernel_stream()) if J is None else fn(C.byref(p), J, tc.kernel_stream())
-    _lib.check(rc)
+    if rc:
+        _lib.check(rc)
 
 
 def k_embed(p: EmbedParams) -> None: _call("stride_k_embed", p)

@@ -10,24 +10,46 @@ from dataclasses import dataclass
 
 import torch
 
-from . import tc
-from .tc import (GemmMat, KvRef, TcGemmResidualParams, TcLmFullParams, TcLmGreedyParams, TcMlp13Params,
-                 TcQkvParams, lanes, mat, ptr)
+from struct import Struct
+
+from . import _lib, tc
+from .tc import KvRef, lanes, mat, ptr
 
 U16 = torch.int16  # bf16 bit patterns travel as int16 tensors
 
+# The parameter blocks (stride_amd._lib's Structures) in packed form: Lanes 4i, GemmMat
+# Q2i, KvRef 56s, pointers Q.
+_EMBED = Struct("<4i3Qi4x").pack
+_NORM = Struct("<4i3Qif").pack
+_QKV = Struct("<4iQQ2iQ2iQ2iQi4x56s3Q2i").pack
+_ATTENTION = Struct("<4iQi4xQi4x56s3Qi4xQ6if4x").pack
+_RESIDUAL = _LM_FULL = Struct("<4iQQ2iQ").pack
+_MLP13 = Struct("<4iQQ2iQ2iQ").pack
+_LM_GREEDY = Struct("<4iQQ2ii4xQ").pack
+
+
+def _check(rc: int) -> None:
+    if rc:
+        _lib.check(rc)
+
+
+def _ptr(t) -> int:
+    return 0 if t is None else t.data_ptr()
+
 
 def gemm_residual(w_tiles, x_tiles, h_tiles, rows: int, r: int = 1, lt: int = 1) -> None:
-    p = TcGemmResidualParams(lanes(rows), ptr(x_tiles), mat(w_tiles), ptr(h_tiles))
-    tc.tc_gemm_residual(p, r, lt)
+    rt, ct = w_tiles.shape[:2]
+    p = _RESIDUAL(rows, (rows + 15) // 16, 0, 0, _ptr(x_tiles), _ptr(w_tiles), rt, ct * 16, _ptr(h_tiles))
+    _check(_lib.packed().stride_tc_gemm_residual(p, r, lt, tc.kernel_stream()))
 
 
 def lm_full(w_tiles, x_tiles, rows: int, out=None):
     T = (rows + 15) // 16
     if out is None:
         out = torch.empty((w_tiles.shape[0], T, 16, 16), dtype=torch.float32, device=x_tiles.device)
-    p = TcLmFullParams(lanes(rows), ptr(x_tiles), mat(w_tiles), ptr(out))
-    tc.tc_lm_full(p, 1)
+    rt, ct = w_tiles.shape[:2]
+    p = _LM_FULL(rows, (rows + 15) // 16, 0, 0, _ptr(x_tiles), _ptr(w_tiles), rt, ct * 16, _ptr(out))
+    _check(_lib.packed().stride_tc_lm_full(p, 1, tc.kernel_stream()))
     return out
 
 
@@ -35,8 +57,11 @@ def mlp13(w1_tiles, w3_tiles, x_tiles, rows: int, out=None, r: int = 1, lt: int 
     T = (rows + 15) // 16
     if out is None:
         out = torch.zeros((T, w1_tiles.shape[0], 16, 16), dtype=U16, device=x_tiles.device)
-    p = TcMlp13Params(lanes(rows), ptr(x_tiles), mat(w1_tiles), mat(w3_tiles), ptr(out))
-    tc.tc_mlp13(p, r, lt)
+    rt, ct = w1_tiles.shape[:2]
+    rt3, ct3 = w3_tiles.shape[:2]
+    p = _MLP13(rows, (rows + 15) // 16, 0, 0, _ptr(x_tiles), _ptr(w1_tiles), rt, ct * 16, _ptr(w3_tiles), rt3, ct3 * 16,
+               _ptr(out))
+    _check(_lib.packed().stride_tc_mlp13(p, r, lt, tc.kernel_stream()))
     return out
 
 
@@ -65,8 +90,9 @@ def best_reset(best: torch.Tensor) -> torch.Tensor:
 def lm_greedy(w_tiles, x_tiles, rows: int, vocab: int, best=None, r: int = 1, lt: int = 1):
     if best is None:
         best = best_init(rows, x_tiles.device)
-    p = TcLmGreedyParams(lanes(rows), ptr(x_tiles), mat(w_tiles), vocab, ptr(best))
-    tc.tc_lm_greedy(p, r, lt)
+    rt, ct = w_tiles.shape[:2]
+    p = _LM_GREEDY(rows, (rows + 15) // 16, 0, 0, _ptr(x_tiles), _ptr(w_tiles), rt, ct * 16, vocab, _ptr(best))
+    _check(_lib.packed().stride_tc_lm_greedy(p, r, lt, tc.kernel_stream()))
     return best
 
 
@@ -170,10 +196,8 @@ def embed(emb_tiles, tokens, rows: int, dim: int, h_out=None):
     lt = (rows + 15) // 16
     if h_out is None:
         h_out = torch.zeros((lt, dim // 16, 16, 16), dtype=torch.float32, device=emb_tiles.device)
-    p = tc.TcEmbedParams()
-    p.l = lanes(rows)
-    p.embed, p.tokens, p.h, p.dim = ptr(emb_tiles), ptr(tokens), ptr(h_out), dim
-    tc.tc_embed(p)
+    p = _EMBED(rows, lt, 0, 0, _ptr(emb_tiles), _ptr(tokens), _ptr(h_out), dim)
+    _check(_lib.packed().stride_tc_embed(p, tc.kernel_stream()))
     return h_out
 
 
@@ -181,11 +205,8 @@ def norm(h_tiles, rows: int, weight, eps: float, per_lane: bool = True, x_out=No
     """tc_norm: bf16 x tiles = RMSNorm(h tiles) * weight."""
     if x_out is None:
         x_out = torch.full(tuple(h_tiles.shape), 0x7FFF, dtype=U16, device=h_tiles.device)
-    p = tc.TcNormParams()
-    p.l = lanes(rows)
-    p.h, p.x, p.weight = ptr(h_tiles), ptr(x_out), ptr(weight)
-    p.dim, p.eps = int(h_tiles.shape[1]) * 16, eps
-    tc.tc_norm(p, per_lane)
+    p = _NORM(rows, (rows + 15) // 16, 0, 0, _ptr(h_tiles), _ptr(x_out), _ptr(weight), h_tiles.shape[1] * 16, eps)
+    _check(_lib.packed().stride_tc_norm(p, 1 if per_lane else 0, tc.kernel_stream()))
     return x_out
 
 
@@ -224,33 +245,26 @@ def attention(q, kv: PagedKv, row_slot, row_pos, n_kv: int, head_dim: int, scale
     if one_kernel:
         if out_tiles is None:
             out_tiles = torch.zeros(((rows + 15) // 16, cols // 16, 16, 16), dtype=U16, device=dev)
-        p = tc.AttentionParams()
-        p.l = lanes(rows)
-        p.q, p.q_stride, p.out, p.out_cols = ptr(q), cols, ptr(out_tiles), cols
-        p.kv = kv.ref
-        p.row_slot, p.row_pos, p.items, p.item_count = ptr(row_slot), ptr(row_pos), None, -1
-        p.scratch, p.max_pages, p.rec_floats = None, max_pages, 4 * head_dim + 8
-        p.layer, p.n_kv, p.n_q, p.head_dim, p.scale = layer, n_kv, 4, head_dim, scale
-        tc.tc_attention(p)
+        _attention(q, rows, cols, out_tiles, kv, row_slot, row_pos, None, -1, None, max_pages, layer, n_kv, head_dim, scale)
         return out_tiles
     if items is None:
         pos = row_pos.cpu().tolist()
         items = torch.tensor([[j, pg] for j in range(rows) for pg in range((pos[j] >> 6) + 1)], dtype=torch.int32,
                              device=dev).reshape(-1)
-    rec = 4 * head_dim + 8
     if scratch is None:
-        scratch = torch.zeros(rows * n_kv * max_pages * rec, dtype=torch.float32, device=dev)
+        scratch = torch.zeros(rows * n_kv * max_pages * (4 * head_dim + 8), dtype=torch.float32, device=dev)
     if out_tiles is None:
         out_tiles = torch.zeros(((rows + 15) // 16, cols // 16, 16, 16), dtype=U16, device=dev)
-    p = tc.AttentionParams()
-    p.l = lanes(rows)
-    p.q, p.q_stride, p.out, p.out_cols = ptr(q), cols, ptr(out_tiles), cols
-    p.kv = kv.ref
-    p.row_slot, p.row_pos, p.items, p.item_count = ptr(row_slot), ptr(row_pos), ptr(items), int(items.numel()) // 2
-    p.scratch, p.max_pages, p.rec_floats = ptr(scratch), max_pages, rec
-    p.layer, p.n_kv, p.n_q, p.head_dim, p.scale = layer, n_kv, 4, head_dim, scale
-    tc.tc_attention(p)
+    _attention(q, rows, cols, out_tiles, kv, row_slot, row_pos, items, items.numel() // 2, scratch, max_pages, layer, n_kv,
+               head_dim, scale)
     return out_tiles
+
+
+def _attention(q, rows, cols, out, kv, row_slot, row_pos, items, count, scratch, max_pages, layer, n_kv, head_dim, scale):
+    p = _ATTENTION(rows, (rows + 15) // 16, 0, 0, _ptr(q), cols, _ptr(out), cols, bytes(kv.ref), _ptr(row_slot),
+                   _ptr(row_pos), _ptr(items), count, _ptr(scratch), max_pages, 4 * head_dim + 8, layer, n_kv, 4, head_dim,
+                   scale)
+    _check(_lib.packed().stride_tc_attention(p, tc.kernel_stream()))
 
 
 def qkv(wq_tiles, wk_tiles, wv_tiles, x_tiles, rows: int, head_dim: int, rope, row_slot, row_pos, kv: PagedKv,
@@ -258,17 +272,9 @@ def qkv(wq_tiles, wk_tiles, wv_tiles, x_tiles, rows: int, head_dim: int, rope, r
     nq = wq_tiles.shape[0] * 16
     if q_out is None:
         q_out = torch.zeros((max(rows, 1), nq), dtype=torch.float32, device=x_tiles.device)
-    p = TcQkvParams()
-    p.l = lanes(rows)
-    p.x = ptr(x_tiles)
-    p.q, p.k, p.v = mat(wq_tiles), mat(wk_tiles), mat(wv_tiles)
-    p.q_out = ptr(q_out)
-    p.q_stride = nq
-    p.kv = kv.ref
-    p.rope = ptr(rope)
-    p.row_slot = ptr(row_slot)
-    p.row_pos = ptr(row_pos)
-    p.layer = layer
-    p.head_dim = head_dim
-    tc.tc_qkv(p)
+    (qt, ct), (kt, kc), (vt, vc) = wq_tiles.shape[:2], wk_tiles.shape[:2], wv_tiles.shape[:2]
+    p = _QKV(rows, (rows + 15) // 16, 0, 0, _ptr(x_tiles), _ptr(wq_tiles), qt, ct * 16, _ptr(wk_tiles), kt, kc * 16,
+             _ptr(wv_tiles), vt, vc * 16, _ptr(q_out), nq, bytes(kv.ref), _ptr(rope), _ptr(row_slot), _ptr(row_pos),
+             layer, head_dim)
+    _check(_lib.packed().stride_tc_qkv(p, tc.kernel_stream()))
     return q_out

@@ -33,6 +33,11 @@ __all__ = [
     "TcCompactParams", "TcEmbedParams", "TcNormParams", "TcGemmF32xParams", "tc_gemm_f32x", "tc_gemm_f32x_noalloc", "tc_embed", "tc_norm", "tc_attention", "tc_compact",
 ]
 
+try:
+    import torch as _torch
+except ImportError:  # parameter blocks and an explicit stream need no torch
+    _torch = None
+
 _stream = None  # None -> torch's current stream at call time
 
 
@@ -46,6 +51,8 @@ def set_kernel_stream(stream) -> None:
 def kernel_stream() -> int:
     s = _stream
     if s is None:
+        if _torch is not None and _torch.cuda.is_initialized():
+            return _torch._C._cuda_getCurrentRawStream(_torch._C._cuda_getDevice())
         import torch
 
         return torch.cuda.current_stream().cuda_stream
