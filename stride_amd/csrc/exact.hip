@@ -643,26 +643,21 @@ __global__ __launch_bounds__(256) void k_exact_norm_lds(StrideNormParams p) {
   for (int r = 0; r < kNormPer; ++r)
     if (tid + 256 * r < items) vsm[tid + 256 * r] = v[r];
   __syncthreads();
-  if (tid < kChains) {
-    float acc[J];
+  // A thread per chain and lane (four lanes in one thread: 6.6 us against 5.9 at 32 rows
+  // of 2048), its LDS reads issued several units ahead.
+  if (tid < kChains * J) {
+    const int t = tid / J, j = tid % J;
+    const float* x = reinterpret_cast<const float*>(vsm) + j;
+    float acc = 0.0f;
+#pragma unroll 4
+    for (int u = t; u < units; u += kChains) {
 #pragma unroll
-    for (int j = 0; j < J; ++j) acc[j] = 0.0f;
-    for (int u = tid; u < units; u += kChains) {
-      if constexpr (J == 1) {
-        const f32x4 x = vsm[u];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[0] = __builtin_fmaf(x[e], x[e], acc[0]);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const f32x4 x = vsm[u * 4 + c];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(x[j], x[j], acc[j]);
-        }
+      for (int c = 0; c < 4; ++c) {
+        const float e = x[(u * 4 + c) * J];
+        acc = __builtin_fmaf(e, e, acc);
       }
     }
-#pragma unroll
-    for (int j = 0; j < J; ++j) part[tid][j] = acc[j];
+    part[t][j] = acc;
   }
   __syncthreads();
   if (tid < J) {

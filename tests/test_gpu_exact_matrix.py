@@ -9,7 +9,7 @@ import torch
 
 from stride_amd import exact as E
 from stride_amd import tc
-from stride_amd._lib import GemmResidualParams, KvRef, LmFullParams, LmGreedyParams, Mlp13Params, QkvParams
+from stride_amd._lib import GemmResidualParams, KvRef, LmFullParams, LmGreedyParams, Mlp13Params, NormParams, QkvParams
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -98,3 +98,22 @@ def test_matrix_qkv(exact, m, hd, kvh):
     assert same(rows[:, 0].reshape(m, -1), rk)
     # V keeps the plain row order of its packed groups: (d0, d0 + 1, d0 + D/2, ...) like K
     assert same(rows[:, 1].reshape(m, -1), rv)
+
+
+@pytest.mark.parametrize("m,dim", [(4, 4), (7, 132), (33, 2048), (2, 4096)])
+def test_norm_rows_equal_single_rows(m, dim):
+    """Four-lane RMSNorm against the same rows one at a time (one lane, whose chains
+    read their LDS items whole), at dims of less than a unit per chain upward."""
+    print("exact norm", m, dim, flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + dim)
+    h, w = torch.randn(m, dim, generator=g, device=DEV) * 3, torch.randn(dim, generator=g, device=DEV)
+    J, _, stride = E.lane_shape(m)
+    hd = E.dim_major(h, stride)
+    out, one = torch.zeros_like(hd), torch.zeros(m, dim, device=DEV)
+    E.k_norm(NormParams(E.lanes(m), tc.ptr(hd), tc.ptr(out), tc.ptr(w), dim, 1e-5), J)
+    for r in range(m):
+        E.k_norm(NormParams(E.lanes(1), tc.ptr(h[r]), tc.ptr(one[r]), tc.ptr(w), dim, 1e-5), 1)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, :m].T.contiguous().view(torch.int32), one.view(torch.int32))
+    want = w.double() * (h.double() / torch.sqrt((h.double() ** 2).mean(1, keepdim=True) + 1e-5))
+    assert torch.allclose(one.double(), want, rtol=2e-6, atol=0)
