@@ -16,6 +16,7 @@
 #include <string>
 
 #include "../../include/stride_exact.h"
+#include "exact_lanes.hpp"
 #include "tc_common.hpp"
 
 namespace stride_tc {
@@ -324,7 +325,8 @@ __global__ __launch_bounds__(64 * WC) void k_exact_gemm_m(typename Op::Params p,
   const int stride = p.l.stride;
   uint32_t xo[2];  // this lane's byte offset from column 0 of a line: columns q and 4 + q
 #pragma unroll
-  for (int s = 0; s < 2; ++s) xo[s] = 4u * (static_cast<uint32_t>(4 * s + q) * stride + min(lg0 * 4 + L * i, stride - L));
+  for (int s = 0; s < 2; ++s)
+    xo[s] = 4u * (static_cast<uint32_t>(4 * s + q) * stride + exact_tile_lane(lg0 * 4 + L * i, p.l.lane_groups, L));
   const int per_chain = (lines + kChains - 1) / kChains;  // lines of chain 0, the longest
   const int nb = (per_chain + NL - 1) / NL;               // batches
 

@@ -71,6 +71,27 @@ def test_matrix_gemms(exact, m, n, k):
     assert np.array_equal(b[:, 1], ri) and np.array_equal(b[:, 0].view(np.uint32), rv.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 64, 264), (18, 4096, 256), (37, 2064, 40), (70, 4096, 48), (130, 3200, 24)])
+def test_lanes_inside_a_wider_buffer(exact, m, n, k):
+    """x as the last lane groups of a wider buffer (it ends with the last live lane):
+    lane, row and stride differ, the bits do not."""
+    print("exact matrix gemm, a run of lanes", m, n, k, flush=True)
+    rng = np.random.default_rng(m + n + k)
+    w, x = bf16(rng, n, k), rng.standard_normal((m, k)).astype(np.float32)
+    J, lane_groups, run = E.lane_shape(m)
+    stride = run + 64
+    wide = dev(np.full((k, stride), np.float32(np.nan)))
+    wide[:, 64:64 + m] = dev(np.ascontiguousarray(x.T))
+    wd = groups(w)
+    out = torch.zeros((wd.shape[0] * 4, stride), device=DEV)
+    l = tc.Lanes(m, lane_groups, stride, 0)
+    E.k_lm_full(LmFullParams(l, tc.ptr(wide) + 4 * 64, E.mat(wd, k), tc.ptr(out) + 4 * 64), J)
+    torch.cuda.synchronize()
+    out = out.cpu().numpy()
+    assert same(out[:n, 64:64 + m].T, exact.gemm(w, x))
+    assert not out[:, :64].any()
+
+
 @pytest.mark.parametrize("m,hd,kvh", [(3, 32, 1), (18, 64, 3), (70, 128, 2)])
 def test_matrix_qkv(exact, m, hd, kvh):
     """q, k and v in one launch: row blocks that straddle the three matrices."""
