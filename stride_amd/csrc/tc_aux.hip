@@ -195,17 +195,6 @@ __global__ __launch_bounds__(64) void k_compact(StrideTcCompactParams p) {
 // ---------------------------------------------------------------------------
 // Attention.
 
-// K or V row of position pos for KV group `group` (src/kernel_common.h:20-25),
-// with the storage page given by the arena geometry.
-template <class KvT>
-__device__ __forceinline__ const KvT* kv_row(const StrideKvRef& kv, int page_shift, int layer, int which, int group,
-                                             int slot, int pos) {
-  const int64_t block = kv.table[static_cast<int64_t>(slot) * kv.max_blocks + (pos >> page_shift)];
-  const int token = pos & ((1 << page_shift) - 1);
-  return static_cast<const KvT*>(kv.arena) + block * kv.block_elems + layer * kv.layer_elems +
-         which * kv.which_elems + group * kv.group_elems + static_cast<int64_t>(token) * kv.head_dim;
-}
-
 // One row's sums over a page, by one wave. Scores: lane i holds position i, and an
 // fmaf chain over the dims in order is a chain of v_mfma_f32_4x4x1_16b_f32, one per dim
 // (one fmaf per output; the query column of four heads is block `dim % 16` of the left
@@ -316,16 +305,28 @@ __device__ __forceinline__ void page_item(const StrideAttentionParams& p, int pa
   const int n = __builtin_amdgcn_readfirstlane(min(visible - p0, kAttnPage));
 
   // Positions past the row's last one are clamped to it (their values are never
-  // used), so every load is unconditional and stays inside the row's own pages.
+  // used), so every load is unconditional and stays inside the row's own pages. Lane i
+  // reads the KV page number of position p0 + i (src/kernel_common.h:20-25), and the
+  // lanes that fetch its V row get it from there, so that two waits come before all of
+  // the page's loads. (With a table read per piece of V the compiler, short of registers
+  // at head_dim 128 in fp32, waited for every V load before the next table read: 64 rows of 2900 positions, 8
+  // groups, 619 us with the combine against 315.)
   const int last = visible - 1;
+  const KvT* base = static_cast<const KvT*>(p.kv.arena) + p.layer * p.kv.layer_elems + g * p.kv.group_elems;
+  const int at = min(p0 + lane, last), in_page = (1 << page_shift) - 1;
+  const int block = p.kv.table[static_cast<int64_t>(slot) * p.kv.max_blocks + (at >> page_shift)];
+  int vblock[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) vblock[k] = __shfl(block, (k * 64 + lane) / (D / kEl));
+  __builtin_amdgcn_sched_barrier(0);  // one wait for them all
   u32x4 vr[kPer], kr[kKey];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int P = k * 64 + lane, i = P / (D / kEl), c = P % (D / kEl);
-    vr[k] = ld_kv(kv_row<KvT>(p.kv, page_shift, p.layer, 1, g, slot, min(p0 + i, last)) + c * kEl);
+    vr[k] = ld_kv(base + vblock[k] * p.kv.block_elems + p.kv.which_elems + (min(p0 + i, last) & in_page) * D + c * kEl);
   }
   {
-    const KvT* key = kv_row<KvT>(p.kv, page_shift, p.layer, 0, g, slot, min(p0 + lane, last));
+    const KvT* key = base + block * p.kv.block_elems + (at & in_page) * D;
 #pragma unroll
     for (int c = 0; c < kKey; ++c) kr[c] = load16(key + kEl * c);
   }

@@ -197,3 +197,24 @@ def test_split_partials_travel_device_coherent():
                 waits = [s for s in ins[before[-1]:a] if s.startswith("s_waitcnt") and "vmcnt(0)" in s]
                 assert waits, f"{name}: arrival atomic not after vmcnt(0)"
     assert seen > 0
+
+
+def test_attention_pages_load_without_waits():
+    """The page kernel issues a page's K and V loads one after the other: a wait for all
+    of them before the last one is issued would make each a memory round trip of its own
+    (the fp32 form at head_dim 128 once waited 32 times)."""
+    path = os.path.join(PKG, "libstride_tc.so")
+    if not os.path.exists(path):
+        pytest.skip("libstride_tc.so not built")
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("llvm-objdump not available")
+    seen = 0
+    for name, ins in functions(disassemble(path)).items():
+        if "k_attn_page" not in name:
+            continue
+        ins = ins[:next(i for i, s in enumerate(ins) if s.startswith("v_mfma"))]
+        loads = [i for i, s in enumerate(ins) if s.startswith("global_load_dwordx4")]
+        waits = [s for s in ins[loads[0]:loads[-1]] if s.startswith("s_waitcnt") and "vmcnt(0)" in s]
+        assert not waits, f"{name}: {len(waits)} waits for every load among the page's {len(loads)} loads"
+        seen += 1
+    assert seen > 0
