@@ -396,6 +396,7 @@ __global__ __launch_bounds__(64 * WC) void k_exact_gemm_m(typename Op::Params p,
       constexpr int m = decltype(ee)::value / R, r = decltype(ee)::value % R;
       aw[wave][m * R * 64 + ((r * LL + pl) * 4 + kp) * NG + pg] = B.a[m][r];
     });
+    wave_phase();  // other lanes' pieces are read from here on
     if (line_of(t, b, 3) < lines) {
       unroll<4>([&](auto n) { slot_step(B, n); });
     } else {
@@ -403,6 +404,7 @@ __global__ __launch_bounds__(64 * WC) void k_exact_gemm_m(typename Op::Params p,
       if (line_of(t, b, 1) < lines) slot_step(B, std::integral_constant<int, 1>{});
       if (line_of(t, b, 2) < lines) slot_step(B, std::integral_constant<int, 2>{});
     }
+    wave_phase();  // the next batch overwrites the slot
   };
   unroll<CH * RT * L>([&](auto ee) {
     constexpr int e = decltype(ee)::value;

@@ -288,11 +288,6 @@ struct PageLds {
   float wt[kHeadsPerGroup * kAttnPage];  // weights [head][position]
   KvT vs[kAttnPage][D];
 };
-__device__ __forceinline__ void wave_phase() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
 template <int D, class KvT>
 __device__ __forceinline__ void page_item(const StrideAttentionParams& p, int page_shift, int j, int page, int g, int lane,
                                           PageLds<D, KvT>& lds) {

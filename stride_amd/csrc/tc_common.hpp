@@ -142,6 +142,15 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Between phases of one wave that exchange data between its lanes through LDS. The
+// hardware performs a wave's LDS accesses in order; this tells the compiler to keep it
+// (no instruction comes of it).
+__device__ __forceinline__ void wave_phase() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 __device__ __forceinline__ float f32_of(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ uint32_t u32_of(float f) { return __float_as_uint(f); }
 
