@@ -92,6 +92,7 @@ struct ResidualOp {  // src/kernels.cu:294-325
   using Params = StrideGemmResidualParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.m.groups; }
+  static int cols(const Params& p) { return p.m.cols; }
   __device__ static const uint16_t* w(const Params& p, int, int group, int& cols) {
     cols = p.m.cols;
     return p.m.w + static_cast<int64_t>(group) * p.m.cols * 4;
@@ -109,6 +110,7 @@ struct Mlp13Op {  // src/kernels.cu:329-363
   using Params = StrideMlp13Params;
   static constexpr int kMats = 2;
   static int groups(const Params& p) { return p.w1.groups; }
+  static int cols(const Params& p) { return p.w1.cols; }
   __device__ static const uint16_t* w(const Params& p, int m, int group, int& cols) {
     const StrideGemmMat& mm = m == 0 ? p.w1 : p.w3;
     cols = mm.cols;
@@ -126,6 +128,7 @@ struct LmFullOp {  // src/kernels.cu:427-452
   using Params = StrideLmFullParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.m.groups; }
+  static int cols(const Params& p) { return p.m.cols; }
   __device__ static const uint16_t* w(const Params& p, int, int group, int& cols) {
     cols = p.m.cols;
     return p.m.w + static_cast<int64_t>(group) * p.m.cols * 4;
@@ -142,6 +145,7 @@ struct LmGreedyOp {  // src/kernels.cu:383-425
   using Params = StrideLmGreedyParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.m.groups; }
+  static int cols(const Params& p) { return p.m.cols; }
   __device__ static const uint16_t* w(const Params& p, int, int group, int& cols) {
     cols = p.m.cols;
     return p.m.w + static_cast<int64_t>(group) * p.m.cols * 4;
@@ -170,6 +174,7 @@ struct QkvOp {  // src/kernels.cu:204-284
   using Params = StrideQkvParams;
   static constexpr int kMats = 1;
   static int groups(const Params& p) { return p.q.groups + 2 * p.k.groups; }
+  static int cols(const Params& p) { return p.q.cols; }
   __device__ static const uint16_t* w(const Params& p, int, int gi, int& cols) {
     const StrideGemmMat& m = gi < p.q.groups ? p.q : (gi < p.q.groups + p.k.groups ? p.k : p.v);
     const int group = gi < p.q.groups ? gi : (gi < p.q.groups + p.k.groups ? gi - p.q.groups : gi - p.q.groups - p.k.groups);
@@ -286,8 +291,8 @@ __global__ __launch_bounds__(64) void k_exact_gemm(typename Op::Params p, int ng
 // larger tiles win where there are enough of them. Against fmaf chains on the vector
 // pipe, same box: N = 3072, K = 2048 at 8 / 32 / 256 rows 11.8 / 16.1 / 65 -> 7.3 /
 // 9.8 / 38 us; 2048 x 8192 34 / 40 / 162 -> 18.1 / 20.0 / 79 us (109 TFLOP/s);
-// 2 x 8192 x 2048 22.6 / 54 / 318 -> 18.1 / 27 / 177 us; 128256 x 2048 at 8 / 32 rows
-// 113 / 354 -> 108 / 184 us.
+// 2 x 8192 x 2048 22.6 / 54 / 318 -> 18.1 / 27 / 177 us; 128256 x 2048 at 32 rows 354
+// -> 184 us.
 template <int N>
 struct FloatsOf;
 template <> struct FloatsOf<1> { typedef float T; };
@@ -478,6 +483,134 @@ __global__ __launch_bounds__(64 * WC) void k_exact_gemm_m(typename Op::Params p,
     if (group < ngroups && lg < p.l.lane_groups)
       Op::template finish<4>(p, group, lg, tid & 15, reinterpret_cast<const float(*)[16]>(ys + k * M * 16));
   }
+}
+
+// Vector form, for up to eight rows of a large weight matrix: two lane groups leave half
+// of a matrix tile's sixteen lanes dead, while here every fmaf is of a live lane (of a
+// dead one for up to four rows). A workgroup of NWV waves runs NB = 2 * NWV reference
+// blocks, i.e. NB consecutive weight groups with the (at most LG) lane groups, so the
+// blocks share x. K is taken kSlice columns at a time: slice s holds line 32 * s + t of chain t,
+// so each lane chains its lines in ascending order and every output's operations are
+// those of chain() (and of the reference). The slice's x is staged once per workgroup in
+// LDS (double buffered, the next slice's loads in flight while the current one is
+// summed), laid out so that lane t's reads of a column are consecutive 16-byte words;
+// each lane loads its own weight line one slice ahead. The matrices of a paired GEMM are
+// swept one after the other, each one's partials folded as in k_exact_gemm.
+// Bound by the vector pipe and, weights from memory, by their stream: 14336 x 8192, 8
+// rows, 42-48 us (4.9-5.6 TB/s) against 51-55 as the best matrix tile of 18.
+constexpr int kSlice = 256;  // 32 lines of 8 columns: one line of each chain
+
+template <class Op, int LG, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_exact_gemm_s(typename Op::Params p, int ngroups) {
+  constexpr int M = Op::kMats;
+  constexpr int NB = 2 * NWV;
+  constexpr int NO = 16;                     // outputs per reference block (4 rows x 4 lanes)
+  constexpr int XS = kSlice * LG;            // staged f32x4 per slice: one per column and lane group
+  constexpr int NT = 64 * NWV;
+  constexpr int XPER = (XS + NT - 1) / NT;   // staging loads per thread
+  __shared__ f32x4 xs[2 * XS];
+  __shared__ float part[NB][kChains][NO * LG];
+  __shared__ float ys[NB][LG][M][16];
+  const int tid = threadIdx.x, wave = tid >> 6, half = (tid >> 5) & 1, t = tid & 31;
+  const int b = wave * 2 + half;
+  const int group = exact_wg_order(blockIdx.x, gridDim.x) * NB + b;
+  const bool live = group < ngroups;
+  const int nlg = p.l.lane_groups;  // at most LG
+
+  // Staging: item q of a slice is column c = q / LG, lane group q % LG (clamped
+  // to the last live one); column 8 * l + e (line l, column e of the line) sits
+  // at (e * 32 + l) * LG + i.
+  f32x4 xr[XPER];
+  auto load_x = [&](int sl) {
+#pragma unroll
+    for (int r = 0; r < XPER; ++r) {
+      const int q = tid + r * NT;
+      if (q < XS) {
+        const int c = q / LG, i = min(q % LG, nlg - 1);
+        xr[r] = *reinterpret_cast<const f32x4*>(p.x + static_cast<int64_t>(sl * kSlice + c) * p.l.stride + 4 * i);
+      }
+    }
+  };
+  auto store_x = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < XPER; ++r) {
+      const int q = tid + r * NT;
+      if (q < XS) {
+        const int c = q / LG, i = q % LG, l = c >> 3, e = c & 7;
+        xs[buf * XS + (e * 32 + l) * LG + i] = xr[r];
+      }
+    }
+  };
+
+  unroll<M>([&](auto mm) {
+    constexpr int m = decltype(mm)::value;
+    int cols = 0;
+    const uint16_t* wg = Op::w(p, m, min(group, ngroups - 1), cols);
+    const int nsl = cols / kSlice;
+    u32x4 wl[2][4];  // this lane's weight line of the current and the next slice
+    auto load_w = [&](int sl, auto buf) {
+      const u32x4* src = reinterpret_cast<const u32x4*>(wg + static_cast<int64_t>(sl * kChains + t) * 32);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) wl[decltype(buf)::value][q] = src[q];
+    };
+    float acc[NO * LG];
+#pragma unroll
+    for (int e = 0; e < NO * LG; ++e) acc[e] = 0.0f;
+    auto step = [&](auto buf) {
+      constexpr int c2 = decltype(buf)::value;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int c = 2 * q + h;  // column c of the line
+          const float wv[4] = {lo_half(wl[c2][q][2 * h]), hi_half(wl[c2][q][2 * h]), lo_half(wl[c2][q][2 * h + 1]),
+                               hi_half(wl[c2][q][2 * h + 1])};
+#pragma unroll
+          for (int i = 0; i < LG; ++i) {
+            const f32x4 xc = xs[c2 * XS + (c * 32 + t) * LG + i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) acc[(i * 4 + r) * 4 + j] = __builtin_fmaf(wv[r], xc[j], acc[(i * 4 + r) * 4 + j]);
+          }
+        }
+      }
+    };
+    load_x(0);
+    load_w(0, std::integral_constant<int, 0>{});
+    store_x(0);
+    __syncthreads();
+    // Slices in pairs so that the register and LDS buffers are compile-time.
+    // The next slice's loads are issued unconditionally (the last slice's again
+    // after it, into buffers nobody reads), so every pass waits on the same loads.
+    int sl = 0;
+    auto one = [&](auto cur) {
+      constexpr int c = decltype(cur)::value;
+      const int nx = min(sl + 1, nsl - 1);
+      load_x(nx);
+      load_w(nx, std::integral_constant<int, c ^ 1>{});
+      step(cur);
+      store_x(c ^ 1);
+      __syncthreads();
+      ++sl;
+    };
+    while (sl < nsl) {
+      one(std::integral_constant<int, 0>{});
+      if (sl < nsl) one(std::integral_constant<int, 1>{});
+    }
+    // Partials of this matrix, folded left to right per output.
+#pragma unroll
+    for (int e = 0; e < NO * LG; ++e) part[b][t][e] = acc[e];
+    __syncthreads();
+    for (int e = t; e < NO * LG; e += kChains) {
+      float y = part[b][0][e];
+      for (int i = 1; i < kChains; ++i) y = y + part[b][i][e];
+      ys[b][e / NO][m][e % NO] = y;
+    }
+    __syncthreads();
+  });
+  if (live)
+    for (int i = 0; i < nlg; ++i) Op::template finish<4>(p, group, i, t, ys[b][i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -750,18 +883,56 @@ int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what
   // 1536 tiles 28.7 at 2 x 2 x 16 waves against 21.3 (128 rows); 2048 tiles 27.2 at
   // 1 x 2 against 25.1 at 2 x 4, whose four lane tiles have to be live (K = 8192: 91
   // against 79); 3072 tiles 48 at 2 x 4 against 38 (256 rows).
-  const int rt = (groups + 3) / 4, lt = (p.l.lane_groups + 3) / 4;
+  const int rt = (groups + 3) / 4, lt = (p.l.lane_groups + 3) / 4, cols = Op::cols(p);
   const int64_t tiles = static_cast<int64_t>(rt) * lt;
-  if (tiles <= 256) return run_matrix<Op, 1, 1, 16, 2, 1>(p, st, what);
+  // Up to eight rows, columns in whole slices: the vector form where it is the faster one.
+  // That is where columns are many (it folds 32 partials of every output and starts fewer
+  // waves), but for row counts that leave its workgroups, 32 rows each and two or three
+  // to a CU, poorly dealt. Measured at 8 rows, 24 sizes up to N = 128256 and K = 8192, each
+  // with its weights in the last-level cache and from memory (the latter second); vector
+  // against the best matrix tile, in us: N = 8192, K = 4096 20.3-22.4 / 18.6-19.5;
+  // 11008 x 3072 20.0-22.2 / 20.2-21.1, x 8192 42.6-45.8 / 47.5-48.3; 14336 x 1024 9.3-12.0
+  // / 10.4-11.3, x 8192 43.4-48.4 / 52.7-54.5; 28672 x 2048 29.4-34.3 / 29.2-30.6;
+  // 36864 x 3072 42-55 / 49-53; 50304 x 1024 28-32 / 30-31, x 2048 44-50 / 49-51; pairs
+  // 2 x 14336 x 1024 18.3-18.5 / 18.4-18.8, x 8192 91-90 / 100-101, 2 x 11008 x 8192
+  // 91-90 / 81-82, 2 x 28672 x 4096 110-109 / 95-101. (An odd number of lines a chain leaves
+  // part of a matrix batch empty: 100000 x 1280 51 / 64.)
+  if (p.l.lane_groups <= 2 && cols % kSlice == 0) {
+    const bool vector = Op::kMats == 2 ? rt >= 832 && rt < 1600 && cols >= 1024
+                                       : (rt > 512 && rt < 832 && cols >= 4096) ||
+                                             (rt >= 832 && rt <= 1536 && cols >= 1024) ||
+                                             (rt >= 2200 && cols >= (cols % (2 * kSlice) == 0 ? 2048 : 768));
+    if (vector) {
+      constexpr int LG = 2, NWV = 4;
+      hipLaunchKernelGGL((k_exact_gemm_s<Op, LG, NWV>), dim3((groups + 2 * NWV - 1) / (2 * NWV)), dim3(64 * NWV), 0, st, p, groups);
+      return launched(what);
+    }
+  }
+  // Few columns leave a wave few lines of each chain: it takes four chains at a time, and
+  // workgroups are half as large (N = 2048, 8 rows: K = 64 3.2 us against 3.8 with sixteen
+  // waves, K = 1024 5.0 / 5.1, K = 2048 7.2 / 7.0).
+  if (tiles <= 256)
+    return cols < 2048 ? run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what) : run_matrix<Op, 1, 1, 16, 2, 1>(p, st, what);
   if constexpr (Op::kMats == 2) {
-    if (lt == 1) return run_matrix<Op, 1, 1, 8, 2, 1>(p, st, what);
+    if (lt == 1)  // 2 x 8192 rows, K = 512: 7.1 us against 7.4; K = 2048 18.6 / 18.3; 2 x 14336, K = 64 7.5 / 8.9
+      return cols < 2048 ? run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what) : run_matrix<Op, 1, 1, 8, 2, 1>(p, st, what);
     if (tiles <= 512) return run_matrix<Op, 1, 2, 16, 1, 1>(p, st, what);
     return run_matrix<Op, 1, 2, 8, 1, 2>(p, st, what);
   } else {
-    // One lane tile over many rows (the vocabulary): the weight stream; 4 x 1 tiles read
-    // it fastest (128256 x 2048, 8 rows: 105-108 us, 5.0 TB/s, against 118 at 2 x 1).
-    if (lt == 1)
-      return tiles >= 2048 ? run_matrix<Op, 4, 1, 4, 2, 1>(p, st, what) : run_matrix<Op, 1, 1, 8, 2, 1>(p, st, what);
+    if (lt == 1) {
+      // One lane tile: the largest row tile that deals the rows about evenly to the CUs (1,
+      // 2 or 4 x 256 row tiles at a time; the sweep above). 4 x 1 reads a vocabulary's
+      // weights fastest (128256 x 2048: 110-112 us against 116 at 2 x 1 and 126 at 1 x 1;
+      // 32000 x 2048 31-32 / 31-35 / 33-36, but 28672 x 1024 18.9-19.3 / 18.3-19.3 /
+      // 17.7-18.7). 2 x 1: N = 8192, K = 1024 6.8-7.8 against 7.3-8.4 at 1 x 1, but
+      // 11008 x 1024 10.3-10.9 / 9.1-9.6. Less than a line for every chain: small
+      // workgroups (32000 x 64: 7.7 us against 8.8).
+      auto dealt = [&](int step) { return (rt + step - 1) / step * step; };
+      if (cols < 8 * kChains && rt > 512) return run_matrix<Op, 1, 1, 4, 4, 1>(p, st, what);
+      if (rt >= 1900 && 20 * dealt(1024) <= 23 * rt) return run_matrix<Op, 4, 1, 4, 2, 1>(p, st, what);
+      if (rt <= 512 || dealt(512) == dealt(256)) return run_matrix<Op, 2, 1, 8, 4, 1>(p, st, what);
+      return run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what);
+    }
     if (tiles <= 512) return run_matrix<Op, 1, 2, 16, 2, 1>(p, st, what);
     if (tiles <= 1024) return run_matrix<Op, 2, 2, 16, 1, 1>(p, st, what);
     if (tiles <= 1536 || (tiles <= 2048 && lt % 4 != 0)) return run_matrix<Op, 1, 2, 8, 1, 2>(p, st, what);

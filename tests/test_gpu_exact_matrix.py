@@ -2,7 +2,7 @@
 the oracle's restatement of the CPU exact path, bit for bit, at the edges of their
 tiles: rows around multiples of 16 and 64, weight groups that leave part of a
 workgroup's rows dead, K of less than one line per chain up to partial last batches,
-and a shape for every tile that the dispatch picks."""
+and a shape for every form that the dispatch picks."""
 import numpy as np
 import pytest
 import torch
@@ -42,7 +42,14 @@ SHAPES = [(2, 64, 8), (5, 100, 264), (16, 4096, 256), (17, 64, 2064),        # u
           (250, 3000, 64)]                                                   # more
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
+# Up to eight rows of many weights: the vector form (whole slices of 256 columns), its
+# last workgroup partly dead; then the forms either side of its lines.
+FEW_ROWS = [(2, 8196, 4096), (5, 14340, 1024), (8, 13320, 1280), (7, 35204, 2048), (3, 8228, 4352),
+            (8, 8192, 4096), (5, 13316, 1032), (9, 8196, 4096), (8, 12292, 264), (6, 35204, 64), (4, 28676, 256),
+            (2, 13316, 3072)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES + FEW_ROWS)
 def test_matrix_gemms(exact, m, n, k):
     print("exact matrix gemm", m, n, k, flush=True)
     rng = np.random.default_rng(m + n + k)
@@ -119,6 +126,12 @@ def test_matrix_qkv(exact, m, hd, kvh):
     assert same(rows[:, 0].reshape(m, -1), rk)
     # V keeps the plain row order of its packed groups: (d0, d0 + 1, d0 + D/2, ...) like K
     assert same(rows[:, 1].reshape(m, -1), rv)
+
+
+@pytest.mark.parametrize("m", [2, 8])
+def test_lanes_inside_a_wider_buffer_vector_form(exact, m):
+    """As above for the vector form, which up to eight rows of many weights take."""
+    test_lanes_inside_a_wider_buffer(exact, m, 8196, 4096)
 
 
 @pytest.mark.parametrize("m,dim", [(4, 4), (7, 132), (33, 2048), (2, 4096)])
