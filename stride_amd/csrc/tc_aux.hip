@@ -648,13 +648,13 @@ __global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_at
         });
         const int n_d = vis_d - p0, end = min(hi - p0, kAttnPage);
         for (int c0 = 4 * whole_steps; c0 < end; c0 += 16) {  // usually once
-          __builtin_amdgcn_wave_barrier();
+          wave_phase();
           unroll<16>([&](auto ee) __attribute__((always_inline)) {
             constexpr int t = decltype(ee)::value / 4, v = decltype(ee)::value % 4;
             const int at = 16 * t + 4 * v + q - c0;
             if (at >= 0 && at < 16) wb[wave][at * 16 + i] = w[t][v];
           });
-          __builtin_amdgcn_wave_barrier();
+          wave_phase();
           for (int pos = c0; pos < min(c0 + 16, end); pos += 4) {
             f32x4 wv[4];
             float vv[4][NDT];

@@ -29,3 +29,14 @@ def test_wave_phase_orders_lds():
     body = body[:body.index("}")]
     assert re.search(r'fence\(__ATOMIC_RELEASE, "wavefront", "local"\).*wave_barrier\(\).*'
                      r'fence\(__ATOMIC_ACQUIRE, "wavefront", "local"\)', body, re.S)
+
+
+def test_attention_tile_tail_weights():
+    """The tile kernel's last positions: lanes store their weights in the wave's wb and
+    read other lanes' (each turn of the loop overwrites them)."""
+    text = source("tc_aux.hip")
+    body = text[text.index("for (int c0 = 4 * whole_steps;"):]
+    body = body[:body.index("auto record =")]
+    kinds = re.findall(r"(wb\[wave\]\[[^;]*\] = )|(&wb\[wave\])|(wave_phase\(\))", body)
+    order = "".join("s" if store else "r" if read else "p" for store, read, _ in kinds)
+    assert order == "pspr", order
