@@ -289,13 +289,11 @@ struct PageLds {
   KvT vs[kAttnPage][D];
 };
 template <int D, class KvT>
-__device__ __forceinline__ void page_item(const StrideAttentionParams& p, int page_shift, int j, int page, int g, int lane,
-                                          PageLds<D, KvT>& lds) {
+__device__ __forceinline__ void page_item(const StrideAttentionParams& p, int page_shift, int j, int slot, int visible, int page,
+                                          int g, int lane, PageLds<D, KvT>& lds) {
   constexpr int kEl = 16 / static_cast<int>(sizeof(KvT));  // elements per 16-byte piece
   constexpr int kPer = kAttnPage * D / kEl / 64;  // pieces of one page of V per lane
   constexpr int kKey = D / kEl;                   // pieces of one K row
-  const int slot = p.row_slot[j];
-  const int visible = p.row_pos[j] + 1;
   const int p0 = page << kAttnPageShift;
   const int n = __builtin_amdgcn_readfirstlane(min(visible - p0, kAttnPage));
 
@@ -361,6 +359,14 @@ __device__ __forceinline__ void page_item(const StrideAttentionParams& p, int pa
 
 // Tiles of kTileRows = 16 consecutive rows (k_attn_tile).
 constexpr int kTileRows = 16;
+
+// Where k_attn_tile tells k_attn_page whether it takes the tile of row j0: the first
+// output of that row, which the combine overwrites after both.
+template <class KvT>
+__device__ __forceinline__ auto* tile_taken(const StrideAttentionParams& p, int j0) {
+  if constexpr (sizeof(KvT) == 4) return static_cast<uint32_t*>(p.out) + j0;
+  else return static_cast<uint16_t*>(p.out) + static_cast<int64_t>(j0 >> 4) * (p.out_cols >> 4) * kTileElems;
+}
 
 // Lane l holds row l % 16: its slot, and its visible positions (0 past the last row).
 struct TileRow {
@@ -430,8 +436,8 @@ __device__ __forceinline__ bool tile_listed(const StrideAttentionParams& p, int 
 // sums at all (a product with a zero weight could turn -0 into +0, or infinity into
 // NaN): a page that is not whole for all of the wave's rows takes whole steps as MFMAs
 // and its last few positions as fmaf under the row's own bound. Tiles whose rows
-// share nothing (decode rows) are left to k_attn_page; a tile whose pages are not all
-// listed is taken item by item.
+// share nothing (decode rows), or whose pages are not all listed, are left to k_attn_page:
+// tile_taken() tells it.
 //
 // Bound by the fp32 units, which the MFMAs (144 of 32 cycles a wave and page) and vector
 // instructions (490 of 4 cycles) take in turn: 82 % of them busy at 2048 rows of one
@@ -453,17 +459,10 @@ __global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_at
     float vs[kAttnPage * D];
     float wb[4][16 * 16];      // a wave's weights of 16 positions
   };
-  constexpr int kItemWaves = 4 * sizeof(PageLds<D, KvT>) <= sizeof(Tile) + 8192 ? 4 : 2;  // waves taking single items
-  union Lds {
-    Tile t;
-    PageLds<D, KvT> item[kItemWaves];
-  };
-  __shared__ __align__(16) unsigned char lds_bytes[sizeof(Lds)];
-  Lds& lds = *reinterpret_cast<Lds*>(lds_bytes);
-  auto& ks = lds.t.ks;
-  auto& vs = lds.t.vs;
-  auto& wb = lds.t.wb;
-  extern __shared__ uint32_t listed[];  // [kTileRows][words] bits, lists that are not the engine's
+  __shared__ __align__(16) Tile lds;
+  auto& ks = lds.ks;
+  auto& vs = lds.vs;
+  auto& wb = lds.wb;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int per_tile = p.n_kv * walkers;
   const int blocks = (p.l.rows + kTileRows - 1) / kTileRows;
@@ -472,25 +471,9 @@ __global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_at
   const int g = blockIdx.x % p.n_kv, walker = static_cast<int>(blockIdx.x) % per_tile / p.n_kv;
   const int rows4 = wave * 4;
   const TileRow tr = tile_row(p, j0, lane);
-  if (!tile_shared(tr)) return;  // k_attn_page takes its items
-  const bool whole = tile_listed(p, j0, lane, tr);
-  if (whole && !__any(walker << kAttnPageShift < tr.visible)) return;
-  if (!whole) {
-    const int nr = min(kTileRows, p.l.rows - j0), words = (p.max_pages + 31) / 32;
-    for (int u = tid; u < kTileRows * words; u += 256) listed[u] = 0u;
-    __syncthreads();
-    for (int u = tid; u < p.item_count; u += 256) {
-      const int r = p.items[2 * u] - j0, c = p.items[2 * u + 1];
-      if (r >= 0 && r < nr && c >= 0 && c < p.max_pages) atomicOr(&listed[r * words + (c >> 5)], 1u << (c & 31));
-    }
-    __syncthreads();
-    if (wave >= kItemWaves) return;
-    for (int c = walker; c < p.max_pages; c += walkers)
-      for (int r = wave; r < nr; r += kItemWaves)
-        if ((listed[r * words + (c >> 5)] >> (c & 31)) & 1u)
-          page_item<D, KvT>(p, page_shift, j0 + r, c, g, lane, lds.item[wave]);
-    return;
-  }
+  const bool taken = tile_shared(tr) && tile_listed(p, j0, lane, tr);
+  if (g == 0 && walker == 0 && tid == 0) *tile_taken<KvT>(p, j0) = taken ? 1 : 0;
+  if (!taken || !__any(walker << kAttnPageShift < tr.visible)) return;
   const float neg_inf = f32_of(0xFF800000u);
   const int i = lane & 15, q = lane >> 4;
 
@@ -523,23 +506,35 @@ __global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_at
     // Staging: piece P = k * 256 + tid of a page is piece P % kRow of position P / kRow;
     // the page numbers of the page after next, and the pieces of the next page, are in
     // flight while a page is summed. Positions past `last` are loaded from it.
-    int blk[kPer];
+    // (Many pieces a thread, fp32 at head_dim 128: a page number a lane, of position `lane`
+    // of the page, that the threads which fetch it get by lane exchange, and positions formed
+    // anew for each page. With numbers and positions for each piece a thread kept some in
+    // scratch memory, and waited for its loads to get them back: 2048 rows of one prompt, 8
+    // groups, 549 us against 440. Few pieces: 226 us against 220 with the exchange.)
+    constexpr bool kOwn = kPer <= 4;
+    int blk[kOwn ? kPer : 1];
     u32x4 kr[kPer], vr[kPer];
     const KvT* base = static_cast<const KvT*>(p.kv.arena) + p.layer * p.kv.layer_elems + g * p.kv.group_elems + (tid % kRow) * kEl;
     const int32_t* table = p.kv.table + static_cast<int64_t>(slot) * p.kv.max_blocks;
-    auto pos_of = [&](int page, int k) { return min((page << kAttnPageShift) + (k * 256 + tid) / kRow, last); };
+    auto pos_of = [&](int page, int at) { return min((page << kAttnPageShift) + at, last); };
     auto load_blk = [&](int page) {
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) blk[k] = table[pos_of(page, k) >> page_shift];
+      for (int k = 0; k < (kOwn ? kPer : 1); ++k) blk[k] = table[pos_of(page, kOwn ? (k * 256 + tid) / kRow : lane) >> page_shift];
     };
     auto fetch = [&](int page) {
+      int at0 = tid / kRow;  // of piece 0, in the page
+      if constexpr (!kOwn) asm volatile("" : "+v"(at0));
+      const int lane_blk = blk[0];
+      if constexpr (!kOwn) load_blk(page + walkers);
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        const KvT* at = base + blk[k] * p.kv.block_elems + (pos_of(page, k) & ((1 << page_shift) - 1)) * D;
-        kr[k] = load16(at);
-        vr[k] = load16(at + p.kv.which_elems);
+        const int at = at0 + k * (256 / kRow);
+        const int64_t block = kOwn ? blk[kOwn ? k : 0] : __shfl(lane_blk, at);
+        const KvT* src = base + block * p.kv.block_elems + (pos_of(page, at) & ((1 << page_shift) - 1)) * D;
+        kr[k] = load16(src);
+        vr[k] = load16(src + p.kv.which_elems);
       }
-      load_blk(page + walkers);
+      if constexpr (kOwn) load_blk(page + walkers);
     };
     auto widen = [&](const u32x4& v, int e) {
       if constexpr (kEl == 8) return f32_of(e & 1 ? v[e >> 1] & 0xFFFF0000u : v[e >> 1] << 16);
@@ -705,9 +700,9 @@ __global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_at
 }
 
 // Items one by one: a wave takes `per_wg` (at most 64) consecutive items of one KV
-// group. TILED: the items of tiles that k_attn_tile takes are skipped. An item outside
-// the record array (page >= max_pages) would write into the next row's records: it is
-// skipped (the caller sizes max_pages for its longest row).
+// group. TILED: those of tiles that k_attn_tile takes are skipped. An item outside the
+// record array (page >= max_pages) would write into the next row's records: it is skipped
+// (the caller sizes max_pages for its longest row).
 template <int D, class KvT, bool TILED>
 __global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int page_shift, int per_wg) {
   __shared__ PageLds<D, KvT> lds;
@@ -715,7 +710,8 @@ __global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int p
   if constexpr (!TILED) {  // per_wg = 1
     const int one = static_cast<int>(blockIdx.x) / p.n_kv;
     const int j = p.items[2 * one], page = p.items[2 * one + 1];
-    if (page >= 0 && page < p.max_pages) page_item<D, KvT>(p, page_shift, j, page, g, lane, lds);
+    if (page >= 0 && page < p.max_pages)
+      page_item<D, KvT>(p, page_shift, j, p.row_slot[j], p.row_pos[j] + 1, page, g, lane, lds);
     return;
   }
   const int item = static_cast<int>(blockIdx.x) / p.n_kv * per_wg + lane;  // this lane's
@@ -724,16 +720,14 @@ __global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int p
     row = p.items[2 * item];
     page = p.items[2 * item + 1];
   }
-  uint64_t todo = __ballot(page >= 0 && page < p.max_pages);
-  for (uint64_t left = todo; left != 0;) {
-    const int j0 = __builtin_amdgcn_readlane(row, __builtin_ctzll(left)) & ~(kTileRows - 1);
-    const uint64_t of_tile = __ballot((row & ~(kTileRows - 1)) == j0);
-    if (tile_shared(tile_row(p, j0, lane))) todo &= ~of_tile;
-    left &= ~of_tile;
-  }
+  const bool valid = page >= 0 && page < p.max_pages && row >= 0 && row < p.l.rows;
+  row = valid ? row : 0;
+  const int slot = p.row_slot[row], visible = p.row_pos[row] + 1;
+  uint64_t todo = __ballot(valid && *tile_taken<KvT>(p, row & ~(kTileRows - 1)) == 0);
   for (; todo != 0; todo &= todo - 1) {
     const int n = __builtin_ctzll(todo);
-    page_item<D, KvT>(p, page_shift, __builtin_amdgcn_readlane(row, n), __builtin_amdgcn_readlane(page, n), g, lane, lds);
+    page_item<D, KvT>(p, page_shift, __builtin_amdgcn_readlane(row, n), __builtin_amdgcn_readlane(slot, n),
+                      __builtin_amdgcn_readlane(visible, n), __builtin_amdgcn_readlane(page, n), g, lane, lds);
   }
 }
 
@@ -1082,8 +1076,7 @@ static int paged(hipStream_t st, const StrideAttentionParams& p, int page_shift)
     // 45 with four, which look at the list for one page each).
     const int tiles = (p.l.rows + kTileRows - 1) / kTileRows * p.n_kv;
     const int walkers = std::max(1, std::min(p.max_pages, 1024 / tiles));
-    const size_t bits = static_cast<size_t>(kTileRows) * ((p.max_pages + 31) / 32) * sizeof(uint32_t);
-    hipLaunchKernelGGL((k_attn_tile<D, KvT>), dim3(tiles * walkers), dim3(256), bits, st, p, page_shift, walkers);
+    hipLaunchKernelGGL((k_attn_tile<D, KvT>), dim3(tiles * walkers), dim3(256), 0, st, p, page_shift, walkers);
     if (int rc = launched("attention (tiles)")) return rc;
     // Where the tiles take everything the waves below only find that out: several items
     // each, but waves enough for decode rows' items.
