@@ -22,6 +22,8 @@ def load():
         lib.mfma_kat_equiv.restype = C.c_int
         lib.mfma_kat_f32.argtypes = [vp, vp, vp, vp, vp, C.c_int32, C.c_int32, vp]
         lib.mfma_kat_f32.restype = C.c_int
+        lib.mfma_kat_4x4.argtypes = lib.mfma_kat_f32.argtypes
+        lib.mfma_kat_4x4.restype = C.c_int
         _lib = lib
     return _lib
 
@@ -44,3 +46,10 @@ def mfma_f32(a, b, c, out, want, steps: int, stream: int) -> None:
                              steps, stream)
     if rc:
         raise RuntimeError(f"mfma_kat_f32 failed ({rc})")
+
+
+def mfma_4x4(a, b, c, out, want, steps: int, stream: int) -> None:
+    rc = load().mfma_kat_4x4(a.data_ptr(), b.data_ptr(), c.data_ptr(), out.data_ptr(), want.data_ptr(), c.shape[0],
+                             steps, stream)
+    if rc:
+        raise RuntimeError(f"mfma_kat_4x4 failed ({rc})")

@@ -3,8 +3,9 @@
 // product): one v_mfma_f32_16x16x32_bf16 per tile on the packed tile layout (the
 // position-invariance test permutes rows and lanes inside a tile), and the
 // equivalence of one 16x16x32 MFMA per 32-column chunk with two chained
-// 32x32x16 MFMAs; and v_mfma_f32_16x16x4_f32 as a chain of fmaf. The gfx950 counterpart of the reference's tc_probe Q1
-// (tools/tc_probe.cu:25-35, 106-139).
+// 32x32x16 MFMAs; and v_mfma_f32_16x16x4_f32 and v_mfma_f32_4x4x1_16b_f32 (one block's
+// left operand given to all sixteen) as chains of fmaf. The gfx950 counterpart of the
+// reference's tc_probe Q1 (tools/tc_probe.cu:25-35, 106-139).
 #include <hip/hip_runtime.h>
 
 #include "../../stride_amd/csrc/tc_common.hpp"
@@ -96,7 +97,45 @@ __global__ __launch_bounds__(256) void k_fma_f32(const float* a, const float* b,
   out[t * 256 + threadIdx.x] = acc;
 }
 
+// out = the accumulator after 16 * steps v_mfma_f32_4x4x1_16b_f32 from c, one workgroup a
+// tile: a [t][4 heads][16 * steps], b [t][16 * steps][64], c and out [t][4][64]. The left
+// operand of step k sits in block k % 16 (lanes 4 * (k % 16) .. + 3, a head each) and is
+// broadcast to the sixteen blocks, whose lanes hold the 64 columns.
+__global__ __launch_bounds__(64) void k_mfma_4x4(const float* a, const float* b, const float* c, float* out, int steps) {
+  const int lane = threadIdx.x;
+  const int64_t t = blockIdx.x;
+  const int kk = 16 * steps;
+  a += t * 4 * kk;
+  b += t * 64 * kk;
+  f32x4 acc;
+  for (int h = 0; h < 4; ++h) acc[h] = c[t * 256 + h * 64 + lane];
+  for (int s = 0; s < steps; ++s) {
+    const float av = a[(lane & 3) * kk + 16 * s + (lane >> 2)];
+    unroll<16>([&](auto kb) {
+      constexpr int k = decltype(kb)::value;
+      acc = __builtin_amdgcn_mfma_f32_4x4x1f32(av, b[(16 * s + k) * 64 + lane], acc, 4, k, 0);
+    });
+  }
+  for (int h = 0; h < 4; ++h) out[t * 256 + h * 64 + lane] = acc[h];
+}
+
+__global__ __launch_bounds__(256) void k_fma_4x4(const float* a, const float* b, const float* c, float* out, int steps) {
+  const int h = threadIdx.x >> 6, lane = threadIdx.x & 63, kk = 16 * steps;
+  const int64_t t = blockIdx.x;
+  float acc = c[t * 256 + threadIdx.x];
+  for (int k = 0; k < kk; ++k) acc = __builtin_fmaf(a[t * 4 * kk + h * kk + k], b[t * 64 * kk + k * 64 + lane], acc);
+  out[t * 256 + threadIdx.x] = acc;
+}
+
 }  // namespace
+
+extern "C" int mfma_kat_4x4(const float* a, const float* b, const float* c, float* out, float* want, int32_t tiles,
+                            int32_t steps, void* stream) {
+  if (!a || !b || !c || !out || !want || tiles <= 0 || steps <= 0) return 1;
+  hipLaunchKernelGGL(k_mfma_4x4, dim3(tiles), dim3(64), 0, static_cast<hipStream_t>(stream), a, b, c, out, steps);
+  hipLaunchKernelGGL(k_fma_4x4, dim3(tiles), dim3(256), 0, static_cast<hipStream_t>(stream), a, b, c, want, steps);
+  return static_cast<int>(hipGetLastError());
+}
 
 extern "C" int mfma_kat_f32(const float* a, const float* b, const float* c, float* out, float* want, int32_t tiles,
                             int32_t steps, void* stream) {

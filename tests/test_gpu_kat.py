@@ -76,6 +76,42 @@ def test_mfma_shapes_equivalent():
         assert torch.equal(o16.view(torch.int32), o32.view(torch.int32)), f"shapes differ at chunks={chunks}"
 
 
+def chain_operands(g, lo, hi):
+    """draw(*shape): normal values over the binary orders lo .. hi, zeros of both signs
+    among them, infinities too in the wide range."""
+    def draw(*shape, scaled=True):
+        t = torch.randn(*shape, generator=g, device=DEV)
+        if scaled:
+            t = torch.ldexp(t, torch.randint(lo, hi, t.shape, generator=g, device=DEV))
+        u = torch.rand(t.shape, generator=g, device=DEV)
+        t[u < 0.02] = 0.0
+        t[u > 0.98] = -0.0
+        if lo == -30:
+            t[(u > 0.5) & (u < 0.502)] = float("inf")
+        return t
+    return draw
+
+
+@pytest.mark.parametrize("lo,hi", [(0, 1), (-30, 30), (-150, -110)])
+def test_f32_4x4_mfma_is_a_chain_of_fmaf(lo, hi):
+    """v_mfma_f32_4x4x1_16b_f32 with each of the sixteen blocks' left operands broadcast in
+    turn equals one fmaf per output, bit for bit: ordinary operands, 60 binary orders of
+    magnitude with infinities, and sums of subnormal products. The scores and mixes of
+    single attention rows rest on this."""
+    g = torch.Generator(device=DEV).manual_seed(11)
+    tiles, steps = 2048, 4
+    draw = chain_operands(g, lo, hi)
+    a, b, c = draw(tiles, 4, 16 * steps), draw(tiles, 16 * steps, 64, scaled=lo >= -30), draw(tiles, 4, 64)
+    out, want = torch.empty_like(c), torch.empty_like(c)
+    kat.mfma_4x4(a, b, c, out, want, steps, stream())
+    torch.cuda.synchronize()
+    if lo == -150:
+        assert ((want != 0) & (want.abs() < 2.0 ** -126)).any()
+    nan = torch.isnan(want)
+    assert torch.equal(nan, torch.isnan(out))
+    assert torch.equal(out.view(torch.int32)[~nan], want.view(torch.int32)[~nan])
+
+
 @pytest.mark.parametrize("lo,hi", [(0, 1), (-30, 30), (-150, -110)])
 def test_f32_mfma_is_a_chain_of_fmaf(lo, hi):
     """v_mfma_f32_16x16x4_f32 equals four fmaf calls, k ascending, bit for bit, for
