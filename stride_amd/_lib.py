@@ -285,8 +285,8 @@ def packed() -> C.CDLL:
     4-11 us of Python per call, more than a small kernel runs; packing takes about 1."""
     global _packed
     if _packed is None:
-        load()
-        lib = C.CDLL(LIB_PATH)  # the same library: function objects with other argument types
+        own = load()  # the same library: function objects with other argument types
+        lib = C.CDLL(own._name, handle=own._handle)
         for name, ints in (("embed", 0), ("norm", 1), ("qkv", 0), ("attention", 0), ("gemm_residual", 2), ("mlp13", 2),
                            ("lm_greedy", 2), ("lm_full", 1)):
             fn = getattr(lib, "stride_tc_" + name)
