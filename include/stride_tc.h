@@ -282,7 +282,9 @@ int stride_tc_norm(const StrideTcNormParams* p, int per_lane, void* stream);
  * max_pages * (12 + 4 * head_dim) floats plus the row's KV page numbers (4 bytes
  * each) and its staging within 159 KiB of LDS: with 16-token KV pages up to 115
  * pages (7360 positions) at head_dim 64, 44 at head_dim 128; item_count == -1
- * beyond that is rejected, item lists beyond it run the page + combine pair.
+ * beyond that is rejected, item lists beyond it run the page + combine pair, for
+ * rows whose records and factors, max_pages * (rec_floats + 4) floats, are at most
+ * 159 KiB (77 pages at head_dim 128); longer ones are rejected.
  * Every row must satisfy row_pos < 64 * max_pages. */
 int stride_tc_attention(const StrideAttentionParams* p, void* stream);
 

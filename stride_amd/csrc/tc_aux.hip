@@ -1034,9 +1034,11 @@ static_assert(offsetof(StrideAttentionParams, kv) == 48 && sizeof(StrideAttentio
 
 static int launched(const char* what);
 
-// LDS that the records of a row may take (the kernel's own static LDS shares the 160
-// KiB, hence the margin).
-constexpr size_t kCombineLdsMax = 159 * 1024;
+// LDS that the one-kernel form may take (160 KiB less a margin). Also the bound on a row's
+// records and page factors in every form, so that what a call may ask for does not depend on
+// the form that takes it (the page kernels and the combine alone would need 32 bytes of LDS
+// a page).
+constexpr size_t kRowLdsMax = 159 * 1024;
 
 // One-kernel attention; its static LDS (staging for up to four waves) and the
 // row's records share the 160 KiB.
@@ -1047,7 +1049,7 @@ constexpr size_t fused_static_lds() {
 
 template <int D, int NWV, bool LIST, class KvT, bool kExact>
 static int fused_nwv(dim3 grid, size_t lds, hipStream_t st, const StrideAttentionParams& p, int page_shift) {
-  if (lds + fused_static_lds<D, NWV, KvT>() > kCombineLdsMax)
+  if (lds + fused_static_lds<D, NWV, KvT>() > kRowLdsMax)
     return fail(STRIDE_TC_EINVAL, "tc_attention: max_pages too large for the one-kernel form (use an item list)");
   static size_t raised = 64 * 1024;
   if (lds > raised) {
@@ -1075,7 +1077,7 @@ static int fused(dim3 grid, size_t lds, hipStream_t st, const StrideAttentionPar
 // larger static staging.)
 template <int D, class KvT = uint16_t>
 static bool fused_fits(size_t lds) {
-  return lds + fused_static_lds<D, 4, KvT>() <= kCombineLdsMax;
+  return lds + fused_static_lds<D, 4, KvT>() <= kRowLdsMax;
 }
 
 // Item-list calls run the one-kernel form (which checks the list on the device)
@@ -1182,8 +1184,8 @@ static int attention(const StrideAttentionParams* p, void* stream, const char* n
   else if (p->l.rows > 0 && (!p->q || !p->out || !p->kv.arena || !p->kv.table || !p->row_slot || !p->row_pos ||
                              (p->item_count >= 0 && !p->scratch) || (p->item_count > 0 && !p->items)))
     why = "missing pointer";
-  else if (static_cast<size_t>(p->max_pages) * (p->rec_floats + kHeadsPerGroup) * sizeof(float) > kCombineLdsMax)
-    why = "max_pages * rec_floats too large for the combine's LDS (159 KiB)";
+  else if (static_cast<size_t>(p->max_pages) * (p->rec_floats + kHeadsPerGroup) * sizeof(float) > kRowLdsMax)
+    why = "a row's records and factors (max_pages * (rec_floats + 4) floats) must fit in 159 KiB";
   if (!why.empty()) return fail(STRIDE_TC_EINVAL, std::string(name) + ": " + why);
   if (p->l.rows == 0) return 0;
   hipStream_t st = static_cast<hipStream_t>(stream);

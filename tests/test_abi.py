@@ -10,7 +10,7 @@ import subprocess
 import pytest
 
 from stride_amd import _lib
-from stride_amd import tc
+from stride_amd import exact, tc
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "stride_tc.h")
@@ -184,3 +184,20 @@ def test_exact_shim_compiles_against_reference_header(tmp_path):
                  "stride::k_lm_greedy(stride::LmGreedyParams const&, int)",
                  "stride::k_lm_full(stride::LmFullParams const&, int)"):
         assert name in syms, name
+
+
+@pytest.mark.parametrize("entry", [tc.tc_attention, exact.k_attention])
+def test_attention_bounds_a_rows_records(entry):
+    """No rows: the checks run, nothing is launched."""
+    p = _lib.AttentionParams()
+    p.kv.group_elems, p.kv.head_dim = 64 * 128, 128
+    p.n_kv, p.n_q, p.head_dim, p.rec_floats, p.out_cols = 1, 4, 128, 520, 512
+    tc.set_kernel_stream(0)
+    try:
+        p.max_pages = 77
+        entry(p)
+        p.max_pages = 78
+        with pytest.raises(tc.StrideTcError, match=r"records and factors .* 159 KiB"):
+            entry(p)
+    finally:
+        tc.set_kernel_stream(None)
