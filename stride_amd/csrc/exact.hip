@@ -885,6 +885,7 @@ int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what
   // against 79); 3072 tiles 48 at 2 x 4 against 38 (256 rows).
   const int rt = (groups + 3) / 4, lt = (p.l.lane_groups + 3) / 4, cols = Op::cols(p);
   const int64_t tiles = static_cast<int64_t>(rt) * lt;
+  auto dealt = [&](int step) { return (rt + step - 1) / step * step; };
   // Up to eight rows, columns in whole slices: the vector form where it is the faster one.
   // That is where columns are many (it folds 32 partials of every output and starts fewer
   // waves), but for row counts that leave its workgroups, 32 rows each and two or three
@@ -896,12 +897,14 @@ int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what
   // 36864 x 3072 42-55 / 49-53; 50304 x 1024 28-32 / 30-31, x 2048 44-50 / 49-51; pairs
   // 2 x 14336 x 1024 18.3-18.5 / 18.4-18.8, x 8192 91-90 / 100-101, 2 x 11008 x 8192
   // 91-90 / 81-82, 2 x 28672 x 4096 110-109 / 95-101. (An odd number of lines a chain leaves
-  // part of a matrix batch empty: 100000 x 1280 51 / 64.)
+  // part of a matrix batch empty: 100000 x 1280 51 / 64. Vocabularies whose 4 x 1 tiles deal
+  // evenly: 128256 x 3072 158 / 155, x 4096 190 / 204; 151936 x 3072 187 / 193.)
   if (p.l.lane_groups <= 2 && cols % kSlice == 0) {
     const bool vector = Op::kMats == 2 ? rt >= 832 && rt < 1600 && cols >= 1024
                                        : (rt > 512 && rt < 832 && cols >= 4096) ||
                                              (rt >= 832 && rt <= 1536 && cols >= 1024) ||
-                                             (rt >= 2200 && cols >= (cols % (2 * kSlice) == 0 ? 2048 : 768));
+                                             (rt >= 2200 && cols >= (cols % (2 * kSlice) == 0 ? 2048 : 768) &&
+                                              !(rt >= 6144 && cols < 4096 && 100 * dealt(1024) <= 103 * rt));
     if (vector) {
       constexpr int LG = 2, NWV = 4;
       hipLaunchKernelGGL((k_exact_gemm_s<Op, LG, NWV>), dim3((groups + 2 * NWV - 1) / (2 * NWV)), dim3(64 * NWV), 0, st, p, groups);
@@ -927,7 +930,6 @@ int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what
       // 17.7-18.7). 2 x 1: N = 8192, K = 1024 6.8-7.8 against 7.3-8.4 at 1 x 1, but
       // 11008 x 1024 10.3-10.9 / 9.1-9.6. Less than a line for every chain: small
       // workgroups (32000 x 64: 7.7 us against 8.8).
-      auto dealt = [&](int step) { return (rt + step - 1) / step * step; };
       if (cols < 8 * kChains && rt > 512) return run_matrix<Op, 1, 1, 4, 4, 1>(p, st, what);
       if (rt >= 1900 && 20 * dealt(1024) <= 23 * rt) return run_matrix<Op, 4, 1, 4, 2, 1>(p, st, what);
       if (rt <= 512 || dealt(512) == dealt(256)) return run_matrix<Op, 2, 1, 8, 4, 1>(p, st, what);
