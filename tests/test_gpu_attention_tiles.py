@@ -73,8 +73,8 @@ def item_list(pos):
 
 
 class Long:
-    """A call on inputs of its own, in both kinds of KV (fp32 of the same values), that
-    has to take the tiles."""
+    """A call on inputs of its own, in both kinds of KV (fp32 of the same values). One of
+    all rows has to take the tiles."""
 
     def __init__(self, seed, slots, pos, hd, page, n_kv=8):
         rng = np.random.default_rng(seed)
@@ -154,6 +154,20 @@ def test_long_lists(exact, case, hd, page):
     m = len(a.pos)
     parts = np.concatenate([a.run(True, rows=(lo, min(lo + 400, m))) for lo in range(0, m, 400)])
     assert np.array_equal(whole.view(np.uint32), parts.view(np.uint32))
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+@pytest.mark.parametrize("n_kv,hd,page", [(2, 64, 16), (1, 128, 64), (1, 32, 32)])
+def test_short_lists_fp32(exact, case, n_kv, hd, page):
+    """The page + combine pair and the one-kernel form over fp32 KV."""
+    print("attention, short list, fp32", case, n_kv, hd, page, flush=True)
+    a = Long(case + hd, *CASES[case], hd, page, n_kv)
+    m = len(a.pos)
+    assert m > 512 and len(a.items) * n_kv <= 32768
+    pair = a.run(True, rows=(0, m))
+    assert np.array_equal(to_bf16(pair), a.want(exact))
+    parts = np.concatenate([a.run(True, rows=(lo, min(lo + 400, m))) for lo in range(0, m, 400)])
+    assert np.array_equal(pair.view(np.uint32), parts.view(np.uint32))
 
 
 @pytest.mark.parametrize("fp32", [False, True])
