@@ -201,8 +201,8 @@ __global__ __launch_bounds__(64) void k_compact(StrideTcCompactParams p) {
 // operand, given to all sixteen blocks, which hold four positions each). Mix: lane d
 // holds dim d, one MFMA per position with the four heads' weights as the column. The
 // four heads cost 8 cycles of the fp32 units a dim or position, against 16 as v_fma_f32.
-// Where the KV loads bound the kernel that shows little (bf16, 128 rows of 4-8 pages 30.1
-// -> 29.4 us), more where they do not (fp32 KV, 32 rows 16.1 -> 13.2 us; bf16, 530 rows of
+// Where the KV loads bound the kernel that does not show (bf16, 128 rows of 4-8 pages, 29-30
+// us either way), more where they do not (fp32 KV, 32 rows 16.1 -> 13.2 us; bf16, 530 rows of
 // 9 pages, each row's read again from L2, 91 -> 69 us).
 //
 // qa: lane h + 4b holds q[h][16e + b] in qa[e].
@@ -302,8 +302,8 @@ __device__ __forceinline__ void page_item(const StrideAttentionParams& p, int pa
   // reads the KV page number of position p0 + i (src/kernel_common.h:20-25), and the
   // lanes that fetch its V row get it from there, so that two waits come before all of
   // the page's loads. (With a table read per piece of V the compiler, short of registers
-  // at head_dim 128 in fp32, waited for every V load before the next table read: 64 rows of 2900 positions, 8
-  // groups, 619 us with the combine against 315.)
+  // at head_dim 128 in fp32, waited for every V load before the next table read: 64 rows
+  // of 2900 positions, 8 groups, 619 us with the combine against 315.)
   const int last = visible - 1;
   const KvT* base = static_cast<const KvT*>(p.kv.arena) + p.layer * p.kv.layer_elems + g * p.kv.group_elems;
   const int at = min(p0 + lane, last), in_page = (1 << page_shift) - 1;
@@ -425,9 +425,9 @@ __device__ __forceinline__ bool tile_listed(const StrideAttentionParams& p, int 
 
 // A tile's pages for one KV group: workgroup (tile, group, walker) takes pages walker,
 // walker + walkers, ... of it and stores the records of page_item. Rows of one sequence
-// share the pages that they read, and there the fmaf chains run as fp32 MFMAs (v_mfma_f32_16x16x4_f32 adds its four products in order, one rounding
-// each: a chain of fmaf, bit for bit), K and V of a page being staged once, widened, for
-// the sixteen rows. A wave holds four rows x four heads as the 16 columns i = 4 * row +
+// share the pages that they read, and there the fmaf chains run as fp32 MFMAs
+// (v_mfma_f32_16x16x4_f32 adds its four products in order, one rounding each: a chain of
+// fmaf, bit for bit), K and V of a page being staged once, widened, for the sixteen rows. A wave holds four rows x four heads as the 16 columns i = 4 * row +
 // head of the score tile (its rows: 16 positions; lane l holds column l % 16). Position
 // 4v + a of a tile is its row 4a + v, so a lane's score register v of quarter a = l / 16
 // is the mix's left operand of step v as it stands: the weights never leave their
@@ -440,9 +440,9 @@ __device__ __forceinline__ bool tile_listed(const StrideAttentionParams& p, int 
 // tile_taken() tells it.
 //
 // Bound by the fp32 units, which the MFMAs (144 of 32 cycles a wave and page) and vector
-// instructions (490 of 4 cycles) take in turn: 82 % of them busy at 2048 rows of one
-// prompt, 8 groups, head_dim 64: 212 us, against 507 us a wave per item on the vector
-// pipe alone.
+// instructions (490 of 4 cycles) take in turn: 81 % of them busy at 2048 rows of one
+// prompt, 8 groups, head_dim 64 (counted): about 215 us, against 507 us a wave per item on
+// the vector pipe alone.
 template <int D, class KvT>
 __global__ __launch_bounds__(256, D == 64 && sizeof(KvT) == 2 ? 3 : 2) void k_attn_tile(StrideAttentionParams p, int page_shift,
                                                                                      int walkers) {
