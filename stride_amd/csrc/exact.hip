@@ -916,6 +916,11 @@ int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what
   // waves, K = 1024 5.0 / 5.1, K = 2048 7.2 / 7.0).
   if (tiles <= 256)
     return cols < 2048 ? run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what) : run_matrix<Op, 1, 1, 16, 2, 1>(p, st, what);
+  // At most a line for every chain: a wave's four chains are one batch, and small workgroups
+  // that fold at once (8192 x 256, 33 rows 7.5 us against 13.5 as below and 12.1 for the
+  // vector form; 3072 x 64 4.7 / 6.8 / 5.3; pairs of 32000 x 128 34 / 62 / 56; of 216 sizes
+  // of more than one lane tile none is slower).
+  if (lt > 1 && cols <= 8 * kChains) return run_matrix<Op, 1, 1, 4, 4, 1>(p, st, what);
   if constexpr (Op::kMats == 2) {
     if (lt == 1)  // 2 x 8192 rows, K = 512: 7.1 us against 7.4; K = 2048 18.6 / 18.3; 2 x 14336, K = 64 7.5 / 8.9
       return cols < 2048 ? run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what) : run_matrix<Op, 1, 1, 8, 2, 1>(p, st, what);
@@ -936,7 +941,8 @@ int run_gemm(const typename Op::Params& p, int J, void* stream, const char* what
       return run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what);
     }
     if (tiles <= 512) return run_matrix<Op, 1, 2, 16, 2, 1>(p, st, what);
-    if (tiles <= 1024) return run_matrix<Op, 2, 2, 16, 1, 1>(p, st, what);
+    if (tiles <= 1024)  // 3072 x 512: 33 rows 6.5 us against 8.0, 64 rows 6.7 / 8.0
+      return cols <= 512 ? run_matrix<Op, 1, 1, 8, 4, 1>(p, st, what) : run_matrix<Op, 2, 2, 16, 1, 1>(p, st, what);
     if (tiles <= 1536 || (tiles <= 2048 && lt % 4 != 0)) return run_matrix<Op, 1, 2, 8, 1, 2>(p, st, what);
     if (tiles <= 2048) return run_matrix<Op, 2, 4, 8, 1, 1>(p, st, what);
     return run_matrix<Op, 2, 2, 4, 2, 1>(p, st, what);

@@ -47,9 +47,11 @@ SHAPES = [(2, 64, 8), (5, 100, 264), (16, 4096, 256), (17, 64, 2064),        # u
 FEW_ROWS = [(2, 8196, 4096), (5, 14340, 1024), (8, 13320, 1280), (7, 35204, 2048), (3, 8228, 4352),
             (8, 8192, 4096), (5, 13316, 1032), (9, 8196, 4096), (8, 12292, 264), (6, 35204, 64), (4, 28676, 256),
             (2, 13316, 3072)]
+# A line or two for every chain at most, more than one lane tile.
+FEW_COLS = [(35, 3076, 512), (17, 4100, 64), (33, 3076, 256), (50, 2052, 8), (250, 4100, 136)]
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES + FEW_ROWS)
+@pytest.mark.parametrize("m,n,k", SHAPES + FEW_ROWS + FEW_COLS)
 def test_matrix_gemms(exact, m, n, k):
     print("exact matrix gemm", m, n, k, flush=True)
     rng = np.random.default_rng(m + n + k)
