@@ -722,8 +722,9 @@ __global__ __launch_bounds__(64) void k_attn_page(StrideAttentionParams p, int p
   }
   const bool valid = page >= 0 && page < p.max_pages && row >= 0 && row < p.l.rows;
   row = valid ? row : 0;
-  const int slot = p.row_slot[row], visible = p.row_pos[row] + 1;
   uint64_t todo = __ballot(valid && *tile_taken<KvT>(p, row & ~(kTileRows - 1)) == 0);
+  if (todo == 0) return;
+  const int slot = p.row_slot[row], visible = p.row_pos[row] + 1;
   for (; todo != 0; todo &= todo - 1) {
     const int n = __builtin_ctzll(todo);
     page_item<D, KvT>(p, page_shift, __builtin_amdgcn_readlane(row, n), __builtin_amdgcn_readlane(slot, n),
@@ -790,8 +791,23 @@ __global__ __launch_bounds__(256) void k_attn_combine(StrideAttentionParams p) {
 #pragma unroll
     for (int c = 0; c < kAhead; ++c)
       if (c < pages) page(c, ahead[u][c]);
-#pragma unroll 8
-    for (int c = kAhead; c < pages; ++c) page(c, recs[c * rf + 8 + hd]);
+    // Eight values in flight, also at the end (the last ones one by one: a row of 74 pages, 2
+    // groups, head_dim 128 18.7 us against 17.7).
+    float v[8];
+    int c0 = kAhead;
+    for (; c0 + 8 <= pages; c0 += 8) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] = recs[(c0 + c) * rf + 8 + hd];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) page(c0 + c, v[c]);
+    }
+    if (c0 < pages) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[c] = recs[min(c0 + c, pages - 1) * rf + 8 + hd];
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if (c0 + c < pages) page(c0 + c, v[c]);
+    }
     const int idx = (g * kHeadsPerGroup + qh) * D + d;
     if constexpr (kExact) static_cast<float*>(p.out)[static_cast<int64_t>(idx) * p.l.stride + j] = acc / dn;
     else out[lane0 + static_cast<int64_t>(idx >> 4) * kTileElems + (idx & 15)] = static_cast<uint16_t>(bf16_rne(acc / dn));
